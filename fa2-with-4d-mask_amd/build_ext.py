@@ -40,13 +40,13 @@ LIB_SAN = BUILD_SAN / "libfa2_4d_mask_hostsan.so"
 HOST_SANITIZE = ["-Xarch_host", "-fsanitize=address", "-Xarch_host", "-fsanitize=undefined",
                  "-Xarch_host", "-fno-sanitize-recover=undefined", "-Xarch_host", "-fno-omit-frame-pointer",
                  "-Xarch_host", "-g"]
-SOURCES = ["fa_fwd.hip", "fa_bwd.hip", "fa_bwd_kv.hip", "fa_bwd_dq.hip", "fa_wide.hip", "fa_mask.hip", "fa_noalloc.hip",
+SOURCES = ["fa_fwd.hip", "fa_bwd.hip", "fa_bwd_kv.hip", "fa_bwd_dq.hip", "fa_wide.hip", "fa_rows.hip", "fa_mask.hip", "fa_noalloc.hip",
            "fa_api.cpp"]
 # Per-file extra flags.  fa_bwd_kv.hip keeps its dK/dV accumulators in AGPRs
 # through inline asm and wants every other MFMA result in VGPRs (read by
-# VALU); fa_wide.hip keeps its MFMA operands in AGPRs and every MFMA result in
-# VGPRs.
-EXTRA_FLAGS = {"fa_bwd_kv.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "fa_wide.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+# VALU); fa_wide.hip and fa_rows.hip (head dim 256) keep their MFMA operands in
+# AGPRs and every MFMA result in VGPRs.
+EXTRA_FLAGS = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for f in ("fa_bwd_kv.hip", "fa_wide.hip", "fa_rows.hip")}
 ARCH = "gfx950"
 
 

@@ -337,6 +337,36 @@ int choose_split(const FaBwdParams* p) {
   return split;
 }
 
+// ---- how the forward runs ----------------------------------------------------
+// Few query rows: the rows of a kv-head's group packed into blocks of 32
+// (fa_rows.hip), which read the mask bytes themselves.  Its work grows with the
+// rows, that of a 256-row block does not, which meets at 64 rows, or 128 where
+// the prepared mask (16 us) is saved too.  Measured at Tk 16384, Hq 32, Hk 8, D
+// 128, in us, this kernel / the 256-row blocks with the key axis split: Tq 32
+// 33 / 63, Tq 64 50 / 65, Tq 128 84 / 68; with a mask Tq 64 61 / 110, Tq 128 104 /
+// 117, Tq 256 186 / 132.
+bool few_rows(const FaFwdParams* p) { return p->seqlen_q <= (p->mask ? 128 : 64); }
+constexpr int kMaxKeySplit = 64;   // fwd_combine_kernel: one range per lane
+struct FwdPlan {
+  bool rows;       // few-rows kernel
+  int split;       // key ranges
+  int64_t bytes;   // workspace of the partial results
+};
+FwdPlan fwd_plan(const FaFwdParams* p) {
+  FwdPlan f{false, 1, 0};
+  const int64_t G = p->heads_q / p->heads_k, R = G * p->seqlen_q, rows = (int64_t)p->batch * p->heads_q * p->seqlen_q;
+  const int64_t keys = p->is_causal ? std::min(p->seqlen_q, p->seqlen_k) : p->seqlen_k;
+  if (few_rows(p)) {
+    f.rows = true;
+    // two workgroups per CU; a range holds at least one tile per wave
+    const int64_t base = (int64_t)p->batch * p->heads_k * ((R + 31) / 32);
+    const int64_t nt = (keys + fa::fwd_rows_keys() - 1) / fa::fwd_rows_keys();
+    f.split = (int)std::max<int64_t>(1, std::min<int64_t>({2 * kCus / base, nt / 4, kMaxKeySplit}));
+  }
+  if (f.split > 1) f.bytes = rows * f.split * (p->head_dim + 2) * (int64_t)sizeof(float);
+  return f;
+}
+
 // The delta workspace holds Delta [B, Hq, Tq], then the LSE the backward
 // kernels read (written by the preprocess).
 float* lse_b_of(const FaBwdParams* p) {
@@ -413,7 +443,8 @@ int fa_fwd(const FaFwdParams* p) {
   if ((st = check_mask_score(p->mask, p->mask_stride_b, p->mask_stride_h, p->mask_stride_q, p->score,
                              p->score_stride_b, p->score_stride_h, p->score_stride_q)))
     return st;
-  if ((st = check_mask_ws(p->mask, p->mask_ws))) return st;
+  const FwdPlan f = fwd_plan(p);
+  if (!f.rows && (st = check_mask_ws(p->mask, p->mask_ws))) return st;
 
   // The forward stages K/V tiles with 32-bit buffer offsets (64 rows of a tile).
   if (p->k_stride_t < 0 || p->k_stride_t >= (1LL << 24) || p->v_stride_t < 0 || p->v_stride_t >= (1LL << 24))
@@ -448,8 +479,33 @@ int fa_fwd(const FaFwdParams* p) {
     a.olsb = p->o_lo_stride_b; a.olst = p->o_lo_stride_t; a.olsh = p->o_lo_stride_h;
   }
   const hipStream_t s = (hipStream_t)p->stream;
+  a.causal = p->is_causal != 0;
+  a.mask4 = (uintptr_t)p->mask % 4 == 0 && p->mask_stride_b % 4 == 0 && p->mask_stride_h % 4 == 0 &&
+            p->mask_stride_q % 4 == 0;
+  a.ns = 1;
+  if (f.split > 1 && p->workspace && p->workspace_bytes >= f.bytes) {
+    if (!aligned16(p->workspace)) return fail(FA_ERR_STRIDE, "workspace must be 16-byte aligned");
+    a.ns = f.split;
+    a.part_o = (float*)p->workspace;
+    a.part_ml = a.part_o + (int64_t)p->batch * p->heads_q * p->seqlen_q * f.split * p->head_dim;
+  }
+  if (f.rows) {
+    if ((st = launch_status(fa::launch_fwd_rows(a, p->head_dim, p->dtype, s), "fa_fwd")) || a.ns == 1) return st;
+    return launch_status(fa::launch_fwd_combine(a, p->head_dim, p->dtype, s), "fa_fwd combine");
+  }
   if (p->head_dim > 128) return launch_status(fa::launch_fwd_wide(a, p->dtype, p->is_causal != 0, s), "fa_fwd");
   return launch_status(fa::launch_fwd(a, p->head_dim, p->dtype, p->is_causal != 0, s), "fa_fwd");
+}
+
+int fa_fwd_plan(const FaFwdParams* p, FaFwdPlan* plan) {
+  if (!p || !plan) return fail(FA_ERR_NULL, "params or plan is NULL");
+  const int st = check_dims(p->batch, p->seqlen_q, p->seqlen_k, p->heads_q, p->heads_k, p->head_dim, p->dtype, p->scale);
+  if (st) return st;
+  const FwdPlan f = fwd_plan(p);
+  plan->needs_mask_ws = f.rows ? 0 : 1;
+  plan->key_split = f.split;
+  plan->workspace_bytes = f.bytes;
+  return FA_OK;
 }
 
 static int check_bwd(const FaBwdParams* p, int split) {

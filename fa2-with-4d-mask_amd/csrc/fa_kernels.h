@@ -109,6 +109,15 @@ struct FwdArgs {
   MaskLayout ml;
   void* olo;            // optional (mask or score): O's rounding residual, dtype, strided like O
   int64_t olsb, olst, olsh;
+  int causal;           // keep j <= i (the few-rows kernel; the others are built for it)
+  int mask4;            // mask rows 4-byte aligned: 32-bit loads allowed (few-rows kernel)
+  // Key split: ns > 1 ranges of the key axis, one workgroup each.  Range i of
+  // row ri = (b Hq + h) Tq + q leaves its O, not divided by its sum, in
+  // part_o[(i rows + ri) D ..] and its running maximum (base 2) and sum in
+  // part_ml[2 (i rows + ri) ..]; fwd_combine_kernel joins them.
+  int ns;
+  float* part_o;
+  float* part_ml;
 };
 
 struct PreArgs {
@@ -199,6 +208,10 @@ struct CvtArgs {
 };
 
 hipError_t launch_fwd(const FwdArgs& a, int D, int dtype, bool causal, hipStream_t s);
+// Few query rows (fa_rows.hip), a.ns key ranges; with a.ns > 1 followed by the combine.
+hipError_t launch_fwd_rows(const FwdArgs& a, int D, int dtype, hipStream_t s);
+hipError_t launch_fwd_combine(const FwdArgs& a, int D, int dtype, hipStream_t s);
+int fwd_rows_keys();
 hipError_t launch_preprocess(const PreArgs& a, int D, int dtype, hipStream_t s);
 hipError_t launch_bwd_dq(const BwdArgs& a, int D, int dtype, bool causal, hipStream_t s);
 // dK/dV of the deterministic path (no dQ), 4 waves x 32 keys per workgroup.

@@ -23,7 +23,7 @@ import torch  # noqa: F401  (must be loaded before the HIP library, see above)
 
 LIB_PATH = (Path(os.environ["FA2_4D_MASK_LIB"]) if os.environ.get("FA2_4D_MASK_LIB")
             else Path(__file__).resolve().parent / "_lib" / "libfa2_4d_mask.so")
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 FA_DTYPE_BF16 = 0
 FA_DTYPE_FP16 = 1
@@ -51,7 +51,17 @@ class FaFwdParams(ctypes.Structure):
         ("is_causal dtype", _i32),
         ("stream mask_ws o_lo", _vp),
         ("o_lo_stride_b o_lo_stride_t o_lo_stride_h", _i64),
+        ("workspace", _vp),
+        ("workspace_bytes", _i64),
     )
+
+
+class FaFwdPlan(ctypes.Structure):
+    _fields_ = [
+        ("needs_mask_ws", _i32),
+        ("key_split", _i32),
+        ("workspace_bytes", _i64),
+    ]
 
 
 class FaBwdParams(ctypes.Structure):
@@ -93,7 +103,7 @@ class FaBwdPlan(ctypes.Structure):
     ]
 
 
-EXPORTED = ("fa_fwd", "fa_bwd_preprocess", "fa_bwd", "fa_bwd_finalize", "fa_bwd_plan", "fa_mask_plan",
+EXPORTED = ("fa_fwd", "fa_fwd_plan", "fa_bwd_preprocess", "fa_bwd", "fa_bwd_finalize", "fa_bwd_plan", "fa_mask_plan",
             "fa_mask_prepare", "fa_last_error", "fa_abi_version", "fa_bwd_noalloc")
 
 _lib = None
@@ -117,6 +127,8 @@ def load_library(path: os.PathLike | None = None) -> ctypes.CDLL:
         lib = ctypes.CDLL(str(p))
         lib.fa_fwd.argtypes = [ctypes.POINTER(FaFwdParams)]
         lib.fa_fwd.restype = ctypes.c_int
+        lib.fa_fwd_plan.argtypes = [ctypes.POINTER(FaFwdParams), ctypes.POINTER(FaFwdPlan)]
+        lib.fa_fwd_plan.restype = ctypes.c_int
         lib.fa_bwd_preprocess.argtypes = [ctypes.POINTER(FaBwdParams)]
         lib.fa_bwd_preprocess.restype = ctypes.c_int
         lib.fa_bwd.argtypes = [ctypes.POINTER(FaBwdParams)]

@@ -222,8 +222,9 @@ def _check_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
 
 def _forward_impl(q, k, v, Mask, Score, scale: float, is_causal: bool, residual: bool = False):
     """Host side of the forward (python/fa2.py:438-488) on logical [B, T, H, D]
-    operands: O [B, Tq, Hq, D], LSE [B, Hq, Tq], the prepared mask (or None)
-    and, with ``residual`` and a mask or a score, O's rounding residual (else
+    operands: O [B, Tq, Hq, D], LSE [B, Hq, Tq], the prepared mask (or None:
+    no mask, or neither the kernels nor, without ``residual``, a backward
+    reads it) and, with ``residual`` and a mask or a score, O's rounding residual (else
     None: the backward then takes Delta from O as stored), plus the operands
     as the kernels saw them (zero-padded to the kernel head dim, see
     ``kernel_head_dim``)."""
@@ -267,7 +268,12 @@ def _forward_impl(q, k, v, Mask, Score, scale: float, is_causal: bool, residual:
             p.dtype = _ext.dtype_code(q.dtype)
             p.stream = _stream(q.device)
             lib = _ext.load_library()
-            if mask is not None:
+            plan = _ext.FaFwdPlan()
+            _ext.check(lib.fa_fwd_plan(ctypes.byref(p), ctypes.byref(plan)), "fa_fwd_plan", lib)
+            if plan.workspace_bytes:
+                ws = torch.empty((plan.workspace_bytes,), dtype=torch.uint8, device=q.device)
+                p.workspace, p.workspace_bytes = ws.data_ptr(), plan.workspace_bytes
+            if mask is not None and (residual or plan.needs_mask_ws):
                 mask_ws = _prepare_mask(mask, mst, B, Hq, Tq, Tk, bool(is_causal), q.device)
                 p.mask_ws = mask_ws.data_ptr()
             _call(lib, "fa_fwd", p)
@@ -292,6 +298,9 @@ def _backward_impl(do, q, k, v, O, LSE, mask, score, mask_ws, mst, sst, scale: f
     if O_lo is not None:
         O_lo = _pad_head_dim(O_lo, D)
     dev = q.device
+    if mask is not None and mask_ws is None and B * Tq * Hq * Tk > 0:
+        # the forward ran without a gradient in sight and read the mask bytes
+        mask_ws = _prepare_mask(mask, mst, B, Hq, Tq, Tk, is_causal, dev)
     dQ = torch.empty((B, Tq, Hq, D), dtype=q.dtype, device=dev)
     dK = torch.empty((B, Tk, Hk, D), dtype=q.dtype, device=dev)
     dV = torch.empty((B, Tk, Hk, D), dtype=q.dtype, device=dev)

@@ -43,12 +43,31 @@ def _mask_ws_bytes(mask: Optional[torch.Tensor], B: int, Hq: int, Tq: int, Tk: i
     return n.value
 
 
+def _fwd_reads_mask_ws(mask, q, k, is_causal: bool) -> bool:
+    """Whether the forward's kernels read the prepared mask (host arithmetic
+    only, as in fa2.py ``_forward_impl``)."""
+    B, Tq, Hq, D = q.shape
+    _, Tk, Hk, _ = k.shape
+    if mask is None or B * Tq * Hq == 0 or Tk == 0:
+        return False
+    lib = _ext.load_library()
+    p = _ext.FaFwdParams()
+    p.mask = 256   # never dereferenced by fa_fwd_plan
+    p.batch, p.seqlen_q, p.seqlen_k, p.heads_q, p.heads_k, p.head_dim = B, Tq, Tk, Hq, Hk, _fa2.kernel_head_dim(D)
+    p.is_causal = 1 if is_causal else 0
+    p.dtype = _ext.dtype_code(q.dtype)
+    plan = _ext.FaFwdPlan()
+    _ext.check(lib.fa_fwd_plan(ctypes.byref(p), ctypes.byref(plan)), "fa_fwd_plan", lib)
+    return bool(plan.needs_mask_ws)
+
+
 @torch.library.custom_op(f"{_NS}::fwd", mutates_args=(), device_types="cuda")
 def fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: Optional[torch.Tensor],
         score: Optional[torch.Tensor], scale: float, is_causal: bool, use_atomic_backward: bool,
         residual: bool) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """O [B, Tq, Hq, D], LSE [B, Hq, Tq] fp32, the prepared mask (uint8, empty
-    without a mask) and O's rounding residual (like O with ``residual`` and a
+    without a mask, and without ``residual`` where the kernels read the mask
+    itself: the backward then prepares it) and O's rounding residual (like O with ``residual`` and a
     mask or a score, else empty), which the backward adds to O for Delta.
     ``use_atomic_backward`` only selects the backward."""
     O, LSE, mask_ws, O_lo, _ = _fa2._forward_impl(q, k, v, mask, score, scale, is_causal, residual)
@@ -69,7 +88,8 @@ def _fwd_fake(q, k, v, mask, score, scale, is_causal, use_atomic_backward, resid
     Tk = k.shape[1]
     O = q.new_empty((B, Tq, Hq, D))
     LSE = q.new_empty((B, Hq, Tq), dtype=torch.float32)
-    ws = q.new_empty((_mask_ws_bytes(mask, B, Hq, Tq, Tk, is_causal),), dtype=torch.uint8)
+    needed = residual or _fwd_reads_mask_ws(mask, q, k, is_causal)
+    ws = q.new_empty((_mask_ws_bytes(mask, B, Hq, Tq, Tk, is_causal) if needed else 0,), dtype=torch.uint8)
     return O, LSE, ws, q.new_empty(_residual_shape(q, mask, score, residual))
 
 

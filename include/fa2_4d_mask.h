@@ -36,7 +36,7 @@
 extern "C" {
 #endif
 
-#define FA_ABI_VERSION 6
+#define FA_ABI_VERSION 7
 
 enum FaDtype { FA_DTYPE_BF16 = 0, FA_DTYPE_FP16 = 1 };
 
@@ -72,12 +72,26 @@ typedef struct FaFwdParams {
   int32_t is_causal;             /* keep j <= i (top-left aligned) */
   int32_t dtype;                 /* enum FaDtype */
   void* stream;                  /* hipStream_t; NULL = default stream */
-  const void* mask_ws;           /* prepared mask (fa_mask_prepare of this mask); required with a mask */
+  const void* mask_ws;           /* prepared mask (fa_mask_prepare of this mask); required with a mask unless
+                                    fa_fwd_plan says that the launch reads the mask itself */
   void* o_lo;                    /* optional [B, Tq, Hq, D] dtype output, written with a mask or a score only:
                                     O's rounding residual (O in fp32 minus O as stored, rounded to dtype),
                                     for fa_bwd_preprocess; NULL = not written */
   int64_t o_lo_stride_b, o_lo_stride_t, o_lo_stride_h;
+  void* workspace;               /* optional: fp32 partial results of the key ranges of a split forward,
+                                    16-byte aligned (fa_fwd_plan gives the size); without it, or with
+                                    less, the key axis is not split */
+  int64_t workspace_bytes;       /* bytes at workspace */
 } FaFwdParams;
+
+/* How fa_fwd runs a problem, so the caller can provide the workspaces. */
+typedef struct FaFwdPlan {
+  int32_t needs_mask_ws;         /* 1: a mask needs its prepared workspace (mask_ws); 0: the launch reads the
+                                    mask bytes themselves (few query rows) and ignores mask_ws */
+  int32_t key_split;             /* ranges the key axis is cut into, when the query rows alone leave CUs
+                                    without a workgroup; 1: not split */
+  int64_t workspace_bytes;       /* size of FaFwdParams.workspace (0 when key_split is 1) */
+} FaFwdPlan;
 
 /* Backward problem.  Reuses the forward's inputs plus O, LSE and dO. */
 typedef struct FaBwdParams {
@@ -183,6 +197,10 @@ int fa_mask_prepare(const FaMaskParams* p);
  * halves, P rounded and its rounding residual (the reference rounds P once,
  * python/fa2.py:128-129); the backward does the same for P and dS. */
 int fa_fwd(const FaFwdParams* p);
+
+/* Fills *plan for the problem in *p (no launch, no GPU access): sizes, head dim,
+ * dtype, causality, and whether mask / score are non-NULL. */
+int fa_fwd_plan(const FaFwdParams* p, FaFwdPlan* plan);
 
 /* Backward preprocess.  Replaces `bwd_preprocess` (python/fa2.py:142-179, launched at
  * python/fa2.py:509-513): delta[b,h,i] = sum_d O*dO in fp32; additionally zeroes the

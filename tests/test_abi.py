@@ -510,3 +510,26 @@ def test_mask_plan_beyond_one_grid_dimension(lib):
                     mask_stride_h=1024, mask_stride_q=32)
     assert lib.fa_mask_plan(ctypes.byref(p), ctypes.byref(nb)) == 2
     assert "32-bit plane indices" in lib.fa_last_error().decode()
+
+
+def test_forward_plan(lib):
+    """Few query rows: no prepared mask, key ranges for two workgroups per CU; the
+    workspace holds each range's fp32 O row, maximum and sum."""
+    ext = _ext()
+
+    def plan(**kw):
+        p = fwd_params(**kw)
+        f = ext.FaFwdPlan()
+        assert lib.fa_fwd_plan(ctypes.byref(p), ctypes.byref(f)) == 0
+        rows = p.batch * p.heads_q * p.seqlen_q
+        assert f.workspace_bytes == (rows * f.key_split * (p.head_dim + 2) * 4 if f.key_split > 1 else 0)
+        return f.needs_mask_ws, f.key_split
+
+    assert plan() == (1, 1)
+    assert plan(seqlen_q=1, seqlen_k=16384) == (0, 64)
+    assert plan(seqlen_q=1, seqlen_k=100) == (0, 1)
+    assert plan(seqlen_q=64, seqlen_k=16384, mask=FAKE) == (0, 8)
+    assert plan(seqlen_q=65)[0] == 1 and plan(seqlen_q=128, mask=FAKE)[0] == 0 and plan(seqlen_q=129, mask=FAKE)[0] == 1
+    assert plan(batch=64, seqlen_q=1, seqlen_k=4096) == (0, 1)
+    # causal rows see no key past the last row
+    assert plan(seqlen_q=4, seqlen_k=16384, is_causal=1) == (0, 1)

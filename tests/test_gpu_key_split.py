@@ -1,0 +1,130 @@
+"""Forward of few query rows (fa_rows.hip) against the eager oracle in float64.
+
+Bound per entry of O: its own rounding to 16 bits, u |O| (half a unit in the
+last place: u = 2^-8 bf16, of 8 significant bits, 2^-11 fp16, of 11); without a
+mask or a score the rounding of P before P V, which moves O by at most
+u sum(p |v|) / sum(p) <= u max|v|; with either P enters in two parts
+(u^2 max|v|); 2^-18 max|v| for fp32 sums, exp2 and the merges' factors.  In fp16
+the parts of a small p are subnormal (steps of 2^-24, so off by 2^-25 each, and
+sum(p) >= 1/2 as the running maximum exceeds no row's by more than one step):
+2^-24 sum|v| more.  LSE (base 2): fp32 dot products of D
+16-bit values, |dlogit| <= D 2^-24 sum|q k| scale log2e < 2e-4 here.
+"""
+
+import ctypes
+import math
+
+import pytest
+import torch
+
+import tilelang_fa2_4d_mask.ops  # noqa: F401  (registers the ops)
+from oracle import eager as E
+
+pytestmark = pytest.mark.gpu
+
+
+def _plan(B, Hq, Hk, D, Tq, Tk, causal, mask, score):
+    from tilelang_fa2_4d_mask import _ext
+
+    lib = _ext.load_library()
+    p = _ext.FaFwdParams()
+    p.batch, p.seqlen_q, p.seqlen_k, p.heads_q, p.heads_k, p.head_dim = B, Tq, Tk, Hq, Hk, D
+    p.is_causal, p.scale = int(causal), 0.1
+    p.mask, p.score = (256 if mask else None), (256 if score else None)
+    plan = _ext.FaFwdPlan()
+    _ext.check(lib.fa_fwd_plan(ctypes.byref(p), ctypes.byref(plan)), "fa_fwd_plan", lib)
+    return plan
+
+
+def _inputs(seed, B, Hq, Hk, D, Tq, Tk, dtype, mask, score):
+    g = torch.Generator().manual_seed(seed)
+    q, k, v = (torch.randn((B, T, H, D), generator=g).to(dtype) for T, H in ((Tq, Hq), (Tk, Hk), (Tk, Hk)))
+    m = s = None
+    if mask == "bernoulli":      # odd row stride (a view): byte loads; one dead row
+        m = (torch.rand((B, Hq, Tq, Tk + 1), generator=g) < 0.6)[..., :Tk]
+        m[0, 0, 0] = False
+    elif mask == "left":         # left padding, per batch entry, broadcast over heads
+        start = torch.tensor([(Tk * (b + 1)) // (B + 1) for b in range(B)]).view(B, 1, 1, 1)
+        m = (torch.arange(Tk) >= start).expand(B, 1, Tq, Tk).contiguous()
+    elif mask == "chunk":
+        m = (torch.arange(Tk) <= torch.arange(Tq)[:, None] + Tk - Tq).view(1, 1, Tq, Tk)
+    if score == "normal":
+        s = torch.randn((B, Hq, Tq, Tk), generator=g)
+    elif score == "padding":     # -inf on the left, one row with nothing else
+        s = torch.where(torch.arange(Tk) >= Tk // 2, 0.0, -math.inf).expand(B, 1, Tq, Tk).clone()
+        s[0, 0, Tq - 1] = -math.inf
+    return q, k, v, m, s
+
+
+def _check(seed, B, Hq, Hk, D, Tq, Tk, dtype, causal, mask, score, scale, residual=False):
+    dev = torch.device("cuda:0")
+    q, k, v, m, s = _inputs(seed, B, Hq, Hk, D, Tq, Tk, dtype, mask, score)
+    dv = [None if x is None else x.to(dev) for x in (q, k, v, m, s)]
+    with torch.no_grad():
+        O, L, ws, lo = torch.ops.tilelang_fa2_4d_mask.fwd(*dv, scale, causal, False, residual)
+    torch.cuda.synchronize()
+    bhsd = [x.transpose(1, 2).double() for x in (q, k, v)]
+    ref = E.eager_ref(*bhsd, m, s, scale=scale, is_causal=causal, compute_dtype=torch.float64).transpose(1, 2)
+    O = O.double().cpu()
+    u = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    two = m is not None or s is not None
+    vmax = v.abs().max().item()
+    assert torch.equal(torch.isnan(O), torch.isnan(ref))
+    fin = ~torch.isnan(ref)
+    sub = 2.0 ** -24 * (1 + v.float().abs().sum(1).max().item()) if dtype == torch.float16 else 0.0
+    bound = u * ref.abs() + ((u * u if two else u) + 2.0 ** -18) * vmax + sub
+    assert bool(((O - ref).abs()[fin] <= bound[fin]).all()), (O - ref).abs()[fin].max().item()
+    if residual and two:
+        both = (O + lo.double().cpu() - ref).abs()
+        # O + residual: the rounding of O itself drops out
+        assert bool((both[fin] <= (u * u * ref.abs() + (u * u + 2.0 ** -18) * vmax + sub)[fin]).all())
+    lse = E.lse2_reference(*bhsd[:2], m, s, scale=scale, is_causal=causal)
+    L = L.double().cpu()
+    dead = ~torch.isfinite(lse)
+    assert torch.equal(torch.isposinf(L), dead)
+    assert (L - lse)[~dead].abs().max().item() < 2e-4
+
+
+ROWS = [
+    # B Hq Hk D Tq Tk dtype causal mask score scale
+    (1, 4, 1, 128, 1, 1, torch.bfloat16, False, None, None, 0.09),
+    (3, 8, 2, 128, 1, 31, torch.bfloat16, False, None, None, 0.09),
+    (2, 8, 8, 64, 1, 4097, torch.float16, False, None, None, 0.125),      # ranges, last tile of one key
+    (1, 32, 1, 128, 2, 2048, torch.bfloat16, False, None, None, -0.09),   # two row blocks
+    (1, 6, 2, 64, 11, 33, torch.float16, True, None, None, 0.125),        # 33 packed rows, causal
+    (2, 4, 2, 128, 64, 64, torch.bfloat16, True, "bernoulli", "normal", 0.09),
+    (4, 8, 2, 128, 1, 3001, torch.bfloat16, False, "left", None, 0.09),
+    (2, 4, 2, 64, 3, 4133, torch.bfloat16, False, "bernoulli", None, 0.125),   # over 32 tiles per wave
+    (1, 4, 2, 128, 128, 1000, torch.float16, False, "chunk", None, 0.09),
+    (2, 4, 4, 128, 1, 2048, torch.bfloat16, False, None, "padding", 0.09),
+    (1, 4, 2, 128, 5, 700, torch.bfloat16, False, "bernoulli", "normal", 0.0),
+    (1, 4, 2, 128, 5, 700, torch.bfloat16, False, None, "normal", -0.09),
+    (1, 4, 1, 256, 1, 2500, torch.bfloat16, False, None, None, 0.06),
+    (2, 4, 2, 256, 17, 300, torch.float16, False, "bernoulli", "normal", 0.06),
+]
+
+
+@pytest.mark.parametrize("case", ROWS, ids=lambda c: f"B{c[0]}H{c[1]}-{c[2]}D{c[3]}T{c[4]}-{c[5]}{c[8] or ''}{c[9] or ''}")
+@pytest.mark.parametrize("residual", [False, True])
+def test_few_rows(cuda, case, residual):
+    B, Hq, Hk, D, Tq, Tk, dtype, causal, mask, score, scale = case
+    plan = _plan(B, Hq, Hk, D, Tq, Tk, causal, mask, score)
+    assert plan.needs_mask_ws == 0
+    print("case", case, "ranges", plan.key_split, flush=True)
+    _check(1, *case, residual=residual)
+
+
+def test_backward_after_a_forward_that_read_the_mask_itself(cuda):
+    """The fwd op without ``residual`` leaves no prepared mask where its kernels
+    read the bytes; the bwd op then prepares it: same gradients as with it."""
+    q, k, v, m, _ = _inputs(3, 2, 4, 2, 64, 40, 500, torch.bfloat16, "bernoulli", None)
+    q, k, v, m = (x.to(cuda) for x in (q, k, v, m))
+    ops = torch.ops.tilelang_fa2_4d_mask
+    O, L, ws, lo = ops.fwd(q, k, v, m, None, 0.125, False, False, False)
+    _, _, ws1, _ = ops.fwd(q, k, v, m, None, 0.125, False, False, True)
+    assert ws.numel() == 0 and ws1.numel() > 0
+    do = torch.randn_like(O)
+    a = ops.bwd(do, q, k, v, O, L, m, None, ws, lo, 0.125, False, False)
+    b = ops.bwd(do, q, k, v, O, L, m, None, ws1, lo, 0.125, False, False)
+    for x, y in zip(a, b):
+        assert torch.equal(x.isnan(), y.isnan()) and torch.equal(x.nan_to_num(), y.nan_to_num())
