@@ -337,6 +337,32 @@ int choose_split(const FaBwdParams* p) {
   return split;
 }
 
+// Key ranges of the 256-row forward: `base` blocks of up to `nt` key tiles each
+// (fewer in causal blocks), one workgroup per CU at a time.  When the blocks
+// alone leave CUs idle, the split with the least estimated time, in us as
+// measured (bf16, Hq 8-32, Tq 256-4096, Tk 1024-16384, mask or not): a workgroup
+// costs 8 plus, per tile, 1.7 (head dim 128) or 1.1 (64), with the two-part P of
+// a mask or score 2.7 or 1.9 -- a quarter less with few CUs busy (clocks) -- and
+// a split adds 6 plus the fp32 partials' way to memory and back.  Tq 512, Tk
+// 8192, Hq 32, D 128: 169 us in one range, 82 in four (102 in two, 101 in six);
+// Tq 1024, Tk 1024, Hq 16: 30 in one, 35-47 in two to eight.
+int fwd_key_split(int64_t base, int64_t nt, int64_t rows, int D, bool prec) {
+  if (base >= kCus) return 1;
+  const double tile = D == 64 ? (prec ? 1.9 : 1.1) : (prec ? 2.7 : 1.7);
+  int best = 1;
+  double best_us = 0;
+  for (int ns = 1; ns <= 16 && ns <= nt; ++ns) {
+    const int64_t wgs = base * ns, rounds = (wgs + kCus - 1) / kCus;
+    const double clk = 0.75 + 0.25 * std::min(1.0, (double)wgs / kCus);
+    double us = rounds * (8 + clk * tile * ((nt + ns - 1) / ns));
+    if (ns > 1) us += 6 + 1.5e-6 * rows * ns * D;
+    if (ns == 1 || us < best_us) {
+      best = ns;
+      best_us = ns == 1 ? 0.95 * us : us;   // split only for a clear gain
+    }
+  }
+  return best;
+}
 // ---- how the forward runs ----------------------------------------------------
 // Few query rows: the rows of a kv-head's group packed into blocks of 32
 // (fa_rows.hip), which read the mask bytes themselves.  Its work grows with the
@@ -362,6 +388,10 @@ FwdPlan fwd_plan(const FaFwdParams* p) {
     const int64_t base = (int64_t)p->batch * p->heads_k * ((R + 31) / 32);
     const int64_t nt = (keys + fa::fwd_rows_keys() - 1) / fa::fwd_rows_keys();
     f.split = (int)std::max<int64_t>(1, std::min<int64_t>({2 * kCus / base, nt / 4, kMaxKeySplit}));
+  } else if (p->head_dim <= 128) {
+    const int64_t base = (int64_t)p->batch * p->heads_q * ((p->seqlen_q + fa::fwd_block_rows() - 1) / fa::fwd_block_rows());
+    const int64_t nt = (keys + fa::kFwdKeys - 1) / fa::kFwdKeys;
+    f.split = fwd_key_split(base, nt, rows, p->head_dim, p->mask || p->score);
   }
   if (f.split > 1) f.bytes = rows * f.split * (p->head_dim + 2) * (int64_t)sizeof(float);
   return f;
@@ -489,8 +519,10 @@ int fa_fwd(const FaFwdParams* p) {
     a.part_o = (float*)p->workspace;
     a.part_ml = a.part_o + (int64_t)p->batch * p->heads_q * p->seqlen_q * f.split * p->head_dim;
   }
-  if (f.rows) {
-    if ((st = launch_status(fa::launch_fwd_rows(a, p->head_dim, p->dtype, s), "fa_fwd")) || a.ns == 1) return st;
+  if (f.rows || a.ns > 1) {
+    const hipError_t e = f.rows ? fa::launch_fwd_rows(a, p->head_dim, p->dtype, s)
+                                : fa::launch_fwd(a, p->head_dim, p->dtype, a.causal, s);
+    if ((st = launch_status(e, "fa_fwd")) || a.ns == 1) return st;
     return launch_status(fa::launch_fwd_combine(a, p->head_dim, p->dtype, s), "fa_fwd combine");
   }
   if (p->head_dim > 128) return launch_status(fa::launch_fwd_wide(a, p->dtype, p->is_causal != 0, s), "fa_fwd");

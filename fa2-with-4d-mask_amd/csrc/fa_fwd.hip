@@ -103,7 +103,9 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
 }
-template <typename T, int D, bool CAUSAL, bool MASK, bool SCORE>
+// SPLIT: the key tiles of each block are cut into a.ns ranges, one workgroup
+// each, which leave fp32 partial results for fwd_combine_kernel (fa_rows.hip).
+template <typename T, int D, bool CAUSAL, bool MASK, bool SCORE, bool SPLIT>
 __global__ __launch_bounds__(kThreads, 1) void fwd_kernel(const FwdArgs a) {
   using V8 = typename Vec8<T>::type;
   constexpr int BM = kBM, BN = kBN;
@@ -146,8 +148,10 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_kernel(const FwdArgs a) {
   // in its L2), and the longest workgroups are dispatched first: rank r is
   // query tile nqt-1-r (causal work grows with the tile), with a mask the
   // tile with the r-th most live key tiles.
-  const int nblk = a.B * a.Hq * a.nqt;
-  const int W = xcd_remap(blockIdx.x, nblk);
+  const int nblk = a.B * a.Hq * a.nqt * (SPLIT ? a.ns : 1);
+  const int W0 = xcd_remap(blockIdx.x, nblk);
+  const int W = SPLIT ? W0 / a.ns : W0;
+  const int sp = SPLIT ? W0 - W * a.ns : 0;   // key range of this workgroup
   const int per_kv = a.G * a.nqt;
   const int bk = W / per_kv;
   const int rem = W - bk * per_kv;
@@ -165,11 +169,22 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_kernel(const FwdArgs a) {
   const int l32 = lane & 31, hf = lane >> 5;
   const int q0 = qt * BM, q0w = q0 + wave * 32;
   const int qrow = q0w + l32;
-  const int Tq = a.Tq, Tk = a.Tk;
+  const int Tq = a.Tq;
+
+  // Key tiles of the workgroup: all of them up to the causal end, or (SPLIT)
+  // range sp of a.ns, of nearly equal counts.  Without a mask a range is taken
+  // as a problem of its own whose key 0 is koff (so Tk, tile and key indices
+  // below count from koff); with a mask the range is one of list positions.
+  const int kv_end = CAUSAL ? min(a.Tk, q0 + BM) : a.Tk;
+  const int nt_all = (kv_end + BN - 1) / BN;
+  const int t_lo = SPLIT && !MASK ? (int)((int64_t)nt_all * sp / a.ns) : 0;
+  const int t_hi = SPLIT && !MASK ? (int)((int64_t)nt_all * (sp + 1) / a.ns) : nt_all;
+  const int koff = t_lo * BN;
+  const int Tk = SPLIT && !MASK ? min(a.Tk, t_hi * BN) - koff : a.Tk;
 
   const T* __restrict__ qp = (const T*)a.q + b * a.qsb + h * a.qsh;
-  const T* __restrict__ kp = (const T*)a.k + b * a.ksb + kvh * a.ksh;
-  const T* __restrict__ vp = (const T*)a.v + b * a.vsb + kvh * a.vsh;
+  const T* __restrict__ kp = (const T*)a.k + b * a.ksb + kvh * a.ksh + (int64_t)koff * a.kst;
+  const T* __restrict__ vp = (const T*)a.v + b * a.vsb + kvh * a.vsh + (int64_t)koff * a.vst;
 
   // ---- Q fragment: lane holds Q[qrow][16 ds + 8 hf + 0..7] -------------------
   V8 qf[QLDS ? 1 : DS];
@@ -194,19 +209,27 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_kernel(const FwdArgs a) {
     flist = (const int32_t*)(a.mws + a.ml.lfwd + pm * a.ml.plfwd) + (int64_t)qt * (1 + a.ml.nft);
     mbits = (const uint32_t*)(a.mws + a.ml.bits + pm * a.ml.pbits) + (int64_t)qrow_c * a.ml.wk;
   }
-  const int kv_end = CAUSAL ? min(Tk, q0 + BM) : Tk;
   // with a mask: count and first two entries in one scalar load (the words
   // past a short list are still inside the workspace; only used when valid)
   int32_t fl[3] = {0, 0, 0};
+  int lb = 0;
   if constexpr (MASK) {
 #pragma unroll
     for (int i = 0; i < 3; ++i) fl[i] = flist[i];
+    if constexpr (SPLIT) {   // positions [pb, pe) of the list
+      const int pb = (int)((int64_t)fl[0] * sp / a.ns), pe = (int)((int64_t)fl[0] * (sp + 1) / a.ns);
+      lb = pb;
+      flist += pb;
+      fl[0] = pe - pb;
+      fl[1] = flist[1];
+      fl[2] = flist[2];
+    }
   }
-  const int nt = MASK ? fl[0] : (kv_end + BN - 1) / BN;
+  const int nt = MASK ? fl[0] : t_hi - t_lo;
   // tiles of this wave (opaque: keeps the per-pair guards dynamic, so that
   // every instantiation gets the same control flow and register assignment);
   // with a mask every wave walks the whole list (causality is applied per key)
-  const int nt_w = (int)opaque((uint32_t)(CAUSAL && !MASK ? min(nt, (min(Tk, q0w + 32) + BN - 1) / BN) : nt));
+  const int nt_w = (int)opaque((uint32_t)(CAUSAL && !MASK ? min(nt, (max(min(Tk, q0w + 32 - koff), 0) + BN - 1) / BN) : nt));
   // List entries: a window of 128 positions sits in two registers (lane i
   // of ents[w] holds position ebase + 64 w + i) and is read with readlane,
   // so that walking the list costs no memory waits in the pipeline; it moves
@@ -217,7 +240,7 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_kernel(const FwdArgs a) {
   int32_t ents[2] = {};   // unused without a mask
   int ebase = 0;
   // range-checked loads (positions past the row read 0): no wait on the count
-  const auto rl = __builtin_amdgcn_make_buffer_rsrc((void*)flist, (short)0, MASK ? (1 + a.ml.nft) * 4 : 0, 0x00020000);
+  const auto rl = __builtin_amdgcn_make_buffer_rsrc((void*)flist, (short)0, MASK ? (1 + a.ml.nft - lb) * 4 : 0, 0x00020000);
   auto fill_ents = [&](int base) __attribute__((always_inline)) {
 #pragma unroll
     for (int w = 0; w < 2; ++w)
@@ -399,7 +422,7 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_kernel(const FwdArgs a) {
   // masked below).  The host keeps the range below 2^32 bytes.
   const int srow0 = min(q0 + 32 * __builtin_amdgcn_readfirstlane(wave), Tq - 1);   // wave-uniform
   const __amdgpu_buffer_rsrc_t srs = __builtin_amdgcn_make_buffer_rsrc(
-      SCORE ? (void*)(a.score + b * a.ssb + h * a.ssh + (int64_t)srow0 * a.ssq) : nullptr, (short)0,
+      SCORE ? (void*)(a.score + b * a.ssb + h * a.ssh + (int64_t)srow0 * a.ssq + koff) : nullptr, (short)0,
       SCORE ? (int)(((int64_t)min(Tq - 1 - srow0, 31) * a.ssq + Tk) * 4) : 0, 0x00020000);
   const uint32_t soff_row = (uint32_t)((int64_t)(qrow_c - srow0) * a.ssq * 4) + hf * 16;
   const float c2 = a.scale_log2;
@@ -586,14 +609,14 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_kernel(const FwdArgs a) {
     if constexpr (SCORE) {
       // (fetched in M(p))
     }
-    const bool edge = (MASK && mpart) || a.zero_scale || (k0 + BN > Tk) || (CAUSAL && k0 + BN - 1 > q0w);
+    const bool edge = (MASK && mpart) || a.zero_scale || (k0 + BN > Tk) || (CAUSAL && k0 + BN - 1 > q0w - koff);
     if (edge) {
       // Keep word of each 32-key half: bit 8 gi + t <-> key k0 + 32 kb +
       // 8 gi + 4 hf + t; keys at or past Tk (causal: past the row) are a
       // suffix of the bit positions.  Each entry then costs a sign-extended
       // bit extract and one bitwise select against -inf (scale 0: against 0
       // for the kept logits, in a copy of its own).
-      const int lim = CAUSAL ? min(Tk, qrow + 1) : Tk;
+      const int lim = CAUSAL ? min(Tk, qrow + 1 - koff) : Tk;
       auto apply = [&](auto ZEROc) __attribute__((always_inline)) {
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
@@ -739,6 +762,26 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_kernel(const FwdArgs a) {
 
   // ---- epilogue: O = acc / l (NaN for a row with no kept key), LSE ----------------
   const float l_tot = half_sum(l_run);
+  if constexpr (SPLIT) {
+    // partial O (not divided by the sum), running maximum and sum of the row
+    if (qrow < Tq) {
+      const int64_t pr = ((int64_t)sp * a.B * a.Hq + (int64_t)b * a.Hq + h) * Tq + qrow;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int gi = 0; gi < 4; ++gi) {
+          f32x4 x;
+#pragma unroll
+          for (int t = 0; t < 4; ++t) x[t] = oacc[nb][gi * 4 + t];
+          *(f32x4*)(a.part_o + pr * D + nb * 32 + gi * 8 + hf * 4) = x;
+        }
+      if (hf == 0) {
+        a.part_ml[2 * pr] = m_run;
+        a.part_ml[2 * pr + 1] = l_tot;
+      }
+    }
+    return;
+  }
   const float inv = 1.0f / l_tot;
   T* os = (T*)smem + wave * 32 * OS;  // wave-private staging, K/V buffers are free now
 #pragma unroll
@@ -805,20 +848,21 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_kernel(const FwdArgs a) {
   }
 }
 
-template <typename T, int D, bool CAUSAL>
+template <typename T, int D, bool CAUSAL, bool SPLIT>
 hipError_t launch_fwd_t(const FwdArgs& a, hipStream_t s) {
-  const dim3 grid((unsigned)(a.B * a.Hq * a.nqt)), block(kThreads);
+  const dim3 grid((unsigned)(a.B * a.Hq * a.nqt * (SPLIT ? a.ns : 1))), block(kThreads);
   const bool m = a.mask != nullptr, sc = a.score != nullptr;
-  if (m && sc) hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, true, true>), grid, block, 0, s, a);
-  else if (m) hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, true, false>), grid, block, 0, s, a);
-  else if (sc) hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, false, true>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, false, false>), grid, block, 0, s, a);
+  if (m && sc) hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, true, true, SPLIT>), grid, block, 0, s, a);
+  else if (m) hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, true, false, SPLIT>), grid, block, 0, s, a);
+  else if (sc) hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, false, true, SPLIT>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, false, false, SPLIT>), grid, block, 0, s, a);
   return hipGetLastError();
 }
 
 template <typename T, int D>
 hipError_t launch_fwd_d(const FwdArgs& a, bool causal, hipStream_t s) {
-  return causal ? launch_fwd_t<T, D, true>(a, s) : launch_fwd_t<T, D, false>(a, s);
+  if (a.ns > 1) return causal ? launch_fwd_t<T, D, true, true>(a, s) : launch_fwd_t<T, D, false, true>(a, s);
+  return causal ? launch_fwd_t<T, D, true, false>(a, s) : launch_fwd_t<T, D, false, false>(a, s);
 }
 
 }  // namespace

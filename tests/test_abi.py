@@ -513,8 +513,9 @@ def test_mask_plan_beyond_one_grid_dimension(lib):
 
 
 def test_forward_plan(lib):
-    """Few query rows: no prepared mask, key ranges for two workgroups per CU; the
-    workspace holds each range's fp32 O row, maximum and sum."""
+    """Few query rows: no prepared mask, key ranges for two workgroups per CU;
+    256-row blocks: split only below one block per CU; the workspace holds each
+    range's fp32 O row, maximum and sum."""
     ext = _ext()
 
     def plan(**kw):
@@ -530,6 +531,8 @@ def test_forward_plan(lib):
     assert plan(seqlen_q=1, seqlen_k=100) == (0, 1)
     assert plan(seqlen_q=64, seqlen_k=16384, mask=FAKE) == (0, 8)
     assert plan(seqlen_q=65)[0] == 1 and plan(seqlen_q=128, mask=FAKE)[0] == 0 and plan(seqlen_q=129, mask=FAKE)[0] == 1
+    assert plan(seqlen_q=512) == (1, 4)
+    assert plan(seqlen_q=512, head_dim=256) == (1, 1)
     assert plan(batch=64, seqlen_q=1, seqlen_k=4096) == (0, 1)
     # causal rows see no key past the last row
     assert plan(seqlen_q=4, seqlen_k=16384, is_causal=1) == (0, 1)

@@ -1,4 +1,5 @@
-"""Forward of few query rows (fa_rows.hip) against the eager oracle in float64.
+"""Forward of few query rows (fa_rows.hip) and of 256-row blocks with the key
+axis split (fa_fwd.hip, SPLIT), against the eager oracle in float64.
 
 Bound per entry of O: its own rounding to 16 bits, u |O| (half a unit in the
 last place: u = 2^-8 bf16, of 8 significant bits, 2^-11 fp16, of 11); without a
@@ -112,6 +113,27 @@ def test_few_rows(cuda, case, residual):
     assert plan.needs_mask_ws == 0
     print("case", case, "ranges", plan.key_split, flush=True)
     _check(1, *case, residual=residual)
+
+
+SPLIT = [
+    (1, 4, 2, 128, 300, 2049, torch.bfloat16, False, None, None, 0.09),     # last range: a tile of one key
+    (2, 4, 2, 64, 257, 1111, torch.float16, False, None, None, 0.125),
+    (1, 2, 1, 128, 1100, 1100, torch.bfloat16, True, None, None, 0.09),     # causal: empty ranges of short blocks
+    (1, 2, 2, 64, 1024, 1024, torch.bfloat16, True, None, "normal", 0.125),
+    (1, 4, 2, 128, 200, 2000, torch.bfloat16, False, "bernoulli", None, 0.09),
+    (1, 4, 2, 128, 200, 2000, torch.float16, False, "chunk", "normal", -0.09),
+    (1, 4, 1, 64, 300, 1500, torch.bfloat16, False, "left", None, 0.125),   # dead leading tiles: short lists
+    (1, 2, 1, 128, 700, 700, torch.bfloat16, True, "bernoulli", None, 0.09),
+]
+
+
+@pytest.mark.parametrize("case", SPLIT, ids=lambda c: f"B{c[0]}H{c[1]}-{c[2]}D{c[3]}T{c[4]}-{c[5]}{c[8] or ''}{c[9] or ''}")
+def test_key_split(cuda, case):
+    B, Hq, Hk, D, Tq, Tk, dtype, causal, mask, score, scale = case
+    plan = _plan(B, Hq, Hk, D, Tq, Tk, causal, mask, score)
+    assert plan.key_split > 1 and plan.needs_mask_ws == 1
+    print("case", case, "ranges", plan.key_split, flush=True)
+    _check(2, *case, residual=True)
 
 
 def test_backward_after_a_forward_that_read_the_mask_itself(cuda):
