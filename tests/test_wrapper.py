@@ -184,3 +184,28 @@ def test_long_rows_are_relaid_head_major():
     # a head-major view of token-major storage is left as it is
     hm = big.transpose(1, 2).contiguous().transpose(1, 2)
     assert fa2._rows_reachable(hm, 540000) is hm
+
+
+def test_float_attention_mask_stays_broadcast(monkeypatch):
+    """A float attention_mask shared by the heads (and the batch) reaches the
+    kernels as one fp32 plane, with the values of mask / scale (+ score)."""
+    import tilelang_fa2_4d_mask.modeling_attention as M
+
+    seen = {}
+
+    def fake(q, k, v, mask, score, *rest):
+        seen.update(mask=mask, score=score)
+        return q
+
+    monkeypatch.setattr(M, "flash_attention_with_4d_mask", fake)
+    q = torch.zeros((2, 4, 5, 64), dtype=torch.bfloat16)
+    for shape in ((2, 1, 5, 5), (1, 1, 5, 5), (2, 4, 5, 5)):
+        am = torch.randn(shape).to(torch.bfloat16)
+        am[..., 3] = torch.finfo(torch.bfloat16).min
+        for given in (None, torch.randn((1, 4, 5, 5))):
+            M.tilelang_flash_attention(q, q, q, attention_mask=am, score=given, scale=0.25)
+            ref = am.float().expand(2, 4, 5, 5) / 0.25
+            ref = ref if given is None else given.expand(2, 4, 5, 5) + ref
+            assert torch.equal(seen["score"], ref) and seen["mask"] is None
+            if given is None:
+                assert [seen["score"].stride(d) == 0 for d in (0, 1)] == [n == 1 for n in shape[:2]]
