@@ -77,6 +77,15 @@ int check_dims(int32_t B, int32_t Tq, int32_t Tk, int32_t Hq, int32_t Hk, int32_
   return FA_OK;
 }
 
+// Columns of the 16-bit operands that exist: head_dim_in, 0 for all of head_dim.
+template <typename P> int columns(const P* p) { return p->head_dim_in ? p->head_dim_in : p->head_dim; }
+template <typename P> int check_columns(const P* p) {
+  if (p->head_dim_in < 0 || p->head_dim_in > p->head_dim || p->head_dim_in % 16)
+    return fail(FA_ERR_HEAD_DIM, "head_dim_in %d must be a multiple of 16 up to head_dim %d (0: head_dim)",
+                p->head_dim_in, p->head_dim);
+  return FA_OK;
+}
+
 int check_mask_score(const uint8_t* mask, int64_t msb, int64_t msh, int64_t msq, const float* score, int64_t ssb,
                      int64_t ssh, int64_t ssq) {
   if (mask && (msb < 0 || msh < 0 || msq < 0)) return fail(FA_ERR_STRIDE, "mask strides must be non-negative");
@@ -462,7 +471,7 @@ const char* fa_last_error(void) { return g_err; }
 int fa_fwd(const FaFwdParams* p) {
   if (!p) return fail(FA_ERR_NULL, "params is NULL");
   int st = check_dims(p->batch, p->seqlen_q, p->seqlen_k, p->heads_q, p->heads_k, p->head_dim, p->dtype, p->scale);
-  if (st) return st;
+  if (st || (st = check_columns(p))) return st;
   if ((st = check_operand("q", p->q, p->q_stride_b, p->q_stride_t, p->q_stride_h))) return st;
   if ((st = check_operand("k", p->k, p->k_stride_b, p->k_stride_t, p->k_stride_h))) return st;
   if ((st = check_operand("v", p->v, p->v_stride_b, p->v_stride_t, p->v_stride_h))) return st;
@@ -496,6 +505,7 @@ int fa_fwd(const FaFwdParams* p) {
   a.ssb = p->score_stride_b; a.ssh = p->score_stride_h; a.ssq = p->score_stride_q;
   a.B = p->batch; a.Tq = p->seqlen_q; a.Tk = p->seqlen_k; a.Hq = p->heads_q; a.Hk = p->heads_k;
   a.G = p->heads_q / p->heads_k;
+  a.Dv = columns(p);
   const int fwd_rows = p->head_dim > 128 ? fa::fwd_wide_block_rows() : fa::fwd_block_rows();
   a.nqt = (p->seqlen_q + fwd_rows - 1) / fwd_rows;
   float sl2b;
@@ -542,7 +552,7 @@ int fa_fwd_plan(const FaFwdParams* p, FaFwdPlan* plan) {
 
 static int check_bwd(const FaBwdParams* p, int split) {
   int st = check_dims(p->batch, p->seqlen_q, p->seqlen_k, p->heads_q, p->heads_k, p->head_dim, p->dtype, p->scale);
-  if (st) return st;
+  if (st || (st = check_columns(p))) return st;
   if ((st = check_operand("q", p->q, p->q_stride_b, p->q_stride_t, p->q_stride_h))) return st;
   if ((st = check_operand("k", p->k, p->k_stride_b, p->k_stride_t, p->k_stride_h))) return st;
   if ((st = check_operand("v", p->v, p->v_stride_b, p->v_stride_t, p->v_stride_h))) return st;
@@ -563,6 +573,10 @@ static int check_bwd(const FaBwdParams* p, int split) {
   const int64_t qspan = (int64_t)(p->seqlen_q + 32) * 2 * (p->q_stride_t > p->do_stride_t ? p->q_stride_t : p->do_stride_t);
   if (qspan >= (1LL << 32))
     return fail(FA_ERR_STRIDE, "seqlen_q * q/dout time stride too large (%lld bytes, the limit is 2^32)", (long long)qspan);
+  // (columns past head_dim_in load from an offset past every record, 2^31)
+  if (columns(p) < p->head_dim && qspan >= (1LL << 31))
+    return fail(FA_ERR_STRIDE, "seqlen_q * q/dout time stride too large for head_dim_in %d (%lld bytes, the limit is 2^31)",
+                p->head_dim_in, (long long)qspan);
   // The dK/dV kernel reads a step's 32 score rows through one buffer with
   // 32-bit offsets, as the forward does a wave's.
   if (p->score && (31 * p->score_stride_q + (int64_t)p->seqlen_k + 64) * 4 >= (1LL << 32))
@@ -633,6 +647,7 @@ int fa_bwd_preprocess(const FaBwdParams* p) {
   a.olo = p->o_lo;
   a.olsb = p->o_lo_stride_b; a.olst = p->o_lo_stride_t; a.olsh = p->o_lo_stride_h;
   a.B = p->batch; a.Tq = p->seqlen_q; a.Hq = p->heads_q; a.Hk = p->heads_k; a.G = p->heads_q / p->heads_k;
+  a.Dv = columns(p);
   a.is_causal = p->is_causal != 0;
   if (p->mask) {
     a.mws = (const char*)p->mask_ws;
@@ -659,6 +674,7 @@ static fa::BwdArgs bwd_args(const FaBwdParams* p, int split) {
   a.ssb = p->score_stride_b; a.ssh = p->score_stride_h; a.ssq = p->score_stride_q;
   a.B = p->batch; a.Tq = p->seqlen_q; a.Tk = p->seqlen_k; a.Hq = p->heads_q; a.Hk = p->heads_k;
   a.G = p->heads_q / p->heads_k;
+  a.Dv = columns(p);
   const int kb = kv_block_keys(p);
   a.nkt = (p->seqlen_k + kb - 1) / kb;
   const int dq_rows_rc = p->head_dim > 128 ? fa::dq_wide_block_rows() : fa::dq_block_rows();
@@ -799,7 +815,7 @@ int fa_bwd_finalize(const FaBwdParams* p) {
     // dq_accum is head-major [B, Hq, Tq, D]
     const int64_t D = p->head_dim, Tq = p->seqlen_q, Hq = p->heads_q;
     fa::CvtArgs c{p->dq_accum, p->dq, p->dq_stride_b, p->dq_stride_t, p->dq_stride_h,
-                  p->batch, p->seqlen_q, p->heads_q, p->head_dim, 1, 0, Hq * Tq * D, D, Tq * D};
+                  p->batch, p->seqlen_q, p->heads_q, columns(p), 1, 0, Hq * Tq * D, D, Tq * D};
     if ((st = launch_status(fa::launch_convert(c, p->dtype, s), "dq convert"))) return st;
   }
   if (split > 1) {
@@ -808,10 +824,10 @@ int fa_bwd_finalize(const FaBwdParams* p) {
     const int64_t slab = (int64_t)p->batch * p->seqlen_k * p->heads_k * p->head_dim;
     const int64_t D = p->head_dim, Tk = p->seqlen_k, Hk = p->heads_k;
     fa::CvtArgs ck{p->dk_accum, p->dk, p->dk_stride_b, p->dk_stride_t, p->dk_stride_h,
-                   p->batch, p->seqlen_k, p->heads_k, p->head_dim, nslab, slab, Tk * Hk * D, Hk * D, D};
+                   p->batch, p->seqlen_k, p->heads_k, columns(p), nslab, slab, Tk * Hk * D, Hk * D, D};
     if ((st = launch_status(fa::launch_convert(ck, p->dtype, s), "dk convert"))) return st;
     fa::CvtArgs cv{p->dv_accum, p->dv, p->dv_stride_b, p->dv_stride_t, p->dv_stride_h,
-                   p->batch, p->seqlen_k, p->heads_k, p->head_dim, nslab, slab, Tk * Hk * D, Hk * D, D};
+                   p->batch, p->seqlen_k, p->heads_k, columns(p), nslab, slab, Tk * Hk * D, Hk * D, D};
     if ((st = launch_status(fa::launch_convert(cv, p->dtype, s), "dv convert"))) return st;
   }
   return FA_OK;

@@ -60,26 +60,27 @@ __global__ __launch_bounds__(256) void preprocess_kernel(const PreArgs a) {
   if (q < a.Tq) {
     const T* op = (const T*)a.o + b * a.osb + (int64_t)q * a.ost + h * a.osh;
     const T* dp = (const T*)a.dout + b * a.dsb + (int64_t)q * a.dst + h * a.dsh;
-#pragma unroll
-    for (int u = 0; u < CPT; ++u) {
-      const int c = part + 4 * u;
-      const auto ov = as_vec8<T>(gload16(op + c * 8));
-      const auto dv = as_vec8<T>(gload16(dp + c * 8));
-#pragma unroll
-      for (int t = 0; t < 8; ++t) acc = fmaf(to_f<T>(ov[t]), to_f<T>(dv[t]), acc);
-    }
-    if (a.olo) {
-      // O's rounding residual from the forward (mask or score): O to about
-      // 16 significant bits
-      const T* lp = (const T*)a.olo + b * a.olsb + (int64_t)q * a.olst + h * a.olsh;
+    // sum over this thread's columns of x dO; the columns all exist (the loads
+    // then go out together) or not
+    auto dot = [&](const T* xp, bool all) __attribute__((always_inline)) {
 #pragma unroll
       for (int u = 0; u < CPT; ++u) {
         const int c = part + 4 * u;
-        const auto lv = as_vec8<T>(gload16(lp + c * 8));
-        const auto dv = as_vec8<T>(gload16(dp + c * 8));
+        const auto xv = as_vec8<T>(all ? gload16(xp + c * 8) : gload16_if(8 * c < a.Dv, xp + c * 8));
+        const auto dv = as_vec8<T>(all ? gload16(dp + c * 8) : gload16_if(8 * c < a.Dv, dp + c * 8));
 #pragma unroll
-        for (int t = 0; t < 8; ++t) acc = fmaf(to_f<T>(lv[t]), to_f<T>(dv[t]), acc);
+        for (int t = 0; t < 8; ++t) acc = fmaf(to_f<T>(xv[t]), to_f<T>(dv[t]), acc);
       }
+    };
+    // O's rounding residual from the forward (mask or score): O to about 16
+    // significant bits
+    const T* lp = (const T*)a.olo + b * a.olsb + (int64_t)q * a.olst + h * a.olsh;
+    if (a.Dv == D) {
+      dot(op, true);
+      if (a.olo) dot(lp, true);
+    } else {
+      dot(op, false);
+      if (a.olo) dot(lp, false);
     }
   }
   acc += __shfl_xor(acc, 1);
@@ -164,8 +165,8 @@ void dq_kernel(const BwdArgs a) {
   if (qrow < Tq) {
 #pragma unroll
     for (int ds = 0; ds < DS; ++ds) {
-      qf[ds] = as_vec8<T>(gload16(qp + (int64_t)qrow * a.qst + ds * 16 + hf * 8));
-      dof[ds] = as_vec8<T>(gload16(dp + (int64_t)qrow * a.dst + ds * 16 + hf * 8));
+      qf[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, qp + (int64_t)qrow * a.qst + ds * 16 + hf * 8));
+      dof[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, dp + (int64_t)qrow * a.dst + ds * 16 + hf * 8));
     }
     lse_q = a.lse[((int64_t)b * a.Hq + h) * Tq + qrow];
     delta_q = a.delta[((int64_t)b * a.Hq + h) * Tq + qrow];
@@ -211,8 +212,9 @@ void dq_kernel(const BwdArgs a) {
       const int idx = tid + u * 256;
       const int r = idx / CH, c = idx % CH;
       const int kk = min(k0 + r, Tk - 1);
-      kreg[u] = gload16(kp + (int64_t)kk * a.kst + c * 8);
-      vreg[u] = gload16(vp + (int64_t)kk * a.vst + c * 8);
+      const int cc = 8 * c < a.Dv ? c : 0;   // (columns that do not exist: zeroed when stored)
+      kreg[u] = gload16(kp + (int64_t)kk * a.kst + cc * 8);
+      vreg[u] = gload16(vp + (int64_t)kk * a.vst + cc * 8);
     }
   };
   auto store_tile = [&](int buf) {
@@ -222,8 +224,8 @@ void dq_kernel(const BwdArgs a) {
     for (int u = 0; u < U; ++u) {
       const int idx = tid + u * 256;
       const int r = idx / CH, c = idx % CH;
-      lds_write16(ks + r * KS + c * 8, kreg[u]);
-      lds_write16(vs + r * VS + c * 8, vreg[u]);
+      lds_write16(ks + r * KS + c * 8, zero_unless(8 * c < a.Dv, kreg[u]));
+      lds_write16(vs + r * VS + c * 8, zero_unless(8 * c < a.Dv, vreg[u]));
     }
   };
 
@@ -339,7 +341,7 @@ void dq_kernel(const BwdArgs a) {
     const int idx = lane + u * 64;
     const int r = idx / CH, c = idx % CH;
     const int qr = q0w + r;
-    if (qr < Tq) gstore16(dqp + (int64_t)qr * a.dqst + c * 8, lds_read16(os + r * OS + c * 8));
+    if (qr < Tq && 8 * c < a.Dv) gstore16(dqp + (int64_t)qr * a.dqst + c * 8, lds_read16(os + r * OS + c * 8));
   }
 }
 

@@ -189,7 +189,7 @@ __global__ __launch_bounds__(NW * 64, 2) void dq_ds_kernel(const BwdArgs a) {
 #pragma unroll
   for (int u = 0; u < UK; ++u) {
     const int idx = tid + u * kDqWaves * 64, r = idx / CH, c = idx % CH;
-    gk[u] = (uint32_t)(r * a.kst * 2 + c * 16);
+    gk[u] = 8 * c < a.Dv ? (uint32_t)(r * a.kst * 2 + c * 16) : kNoRec;
     swk[u] = opaque(lds0 + r * ROWB + ((c ^ swz_q<D>(r)) * 16));
   }
   // staging chunk u' (bytes lane 16 + u' 1024 of a tile) = chunk lane/32 + 2 u' of key lane%32
@@ -228,7 +228,7 @@ __global__ __launch_bounds__(NW * 64, 2) void dq_ds_kernel(const BwdArgs a) {
       }
     }
     const int rows = inr ? min(32, Tk - kb * 32) : 0;
-    const int nrec = rows > 0 ? (int)((int64_t)(rows - 1) * a.kst * 2 + ROWB) : 0;
+    const int nrec = rows > 0 ? (int)((int64_t)(rows - 1) * a.kst * 2 + 2 * a.Dv) : 0;
     const auto rk = __builtin_amdgcn_make_buffer_rsrc((void*)(kbase + (int64_t)kb * 32 * a.kst), (short)0, nrec, 0x00020000);
 #pragma unroll
     for (int u = 0; u < UK; ++u) stk[S][u] = __builtin_amdgcn_raw_buffer_load_b128(rk, gk[u], 0, 0);
@@ -358,7 +358,7 @@ __global__ __launch_bounds__(NW * 64, 2) void dq_ds_kernel(const BwdArgs a) {
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
       const int idx = lane + u * 64, r = idx / CH, c = idx % CH;
-      if (q0 + r < Tq) gstore16(dqp + (int64_t)(q0 + r) * a.dqst + c * 8, ov[u]);
+      if (q0 + r < Tq && 8 * c < a.Dv) gstore16(dqp + (int64_t)(q0 + r) * a.dqst + c * 8, ov[u]);
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }

@@ -107,7 +107,7 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
   const int key = kw0 + l32;              // this lane's key (column of S)
   const int kc = min(key, Tk - 1);
   // scale == 0: every kept logit is 0, i.e. P = exp2(-LSE2): a zero multiplier
-  const float c2 = a.zero_scale ? 0.f : a.scale_log2, scale = a.scale;
+  const float c2 = a.zero_scale ? 0.f : a.scale_log2;
 
   const T* __restrict__ kp = (const T*)a.k + b * a.ksb + kvh * a.ksh;
   const T* __restrict__ vp = (const T*)a.v + b * a.vsb + kvh * a.vsh;
@@ -118,8 +118,8 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
   V8 kf[DS], vf[DS];
 #pragma unroll
   for (int ds = 0; ds < DS; ++ds) {
-    kf[ds] = as_vec8<T>(gload16(kp + (int64_t)kc * a.kst + ds * 16 + hf * 8));
-    vf[ds] = as_vec8<T>(gload16(vp + (int64_t)kc * a.vst + ds * 16 + hf * 8));
+    kf[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, kp + (int64_t)kc * a.kst + ds * 16 + hf * 8));
+    vf[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, vp + (int64_t)kc * a.vst + ds * 16 + hf * 8));
   }
   // The fragments stay in AGPRs for the whole loop (MFMA reads its A and B
   // operands from AGPRs as well): 64 VGPRs freed, which the masked and score
@@ -254,8 +254,8 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
 #pragma unroll
   for (int u = 0; u < UQ; ++u) {
     const int idx = tid + u * kKvWaves * 64, r = idx / CH, c = idx % CH;
-    gq[u] = (uint32_t)(r * a.qst * 2 + c * 16);
-    gd[u] = (uint32_t)(r * a.dst * 2 + c * 16);
+    gq[u] = 8 * c < a.Dv ? (uint32_t)(r * a.qst * 2 + c * 16) : kNoRec;
+    gd[u] = 8 * c < a.Dv ? (uint32_t)(r * a.dst * 2 + c * 16) : kNoRec;
     sw[u] = opaque(lds0 + r * ROWB + ((c ^ swz_q<D>(r)) * 16));
     if constexpr (SIX) sw2[u] = opaque(sw[u] + kHi);
   }
@@ -268,8 +268,8 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
   // range check includes, so rows past Tq read as zeros.  Padding steps use
   // descriptors without records.  State: next tile ld_it (head ld_h, first
   // row ld_qs), scalar byte offsets of that row in Q, dO and LSE/Delta.
-  const uint32_t q_rec = (uint32_t)((int64_t)(Tq - 1) * a.qst * 2 + ROWB);
-  const uint32_t d_rec = (uint32_t)((int64_t)(Tq - 1) * a.dst * 2 + ROWB);
+  const uint32_t q_rec = (uint32_t)((int64_t)(Tq - 1) * a.qst * 2 + 2 * a.Dv);
+  const uint32_t d_rec = (uint32_t)((int64_t)(Tq - 1) * a.dst * 2 + 2 * a.Dv);
   const uint32_t inc_q = (uint32_t)(kStep * a.qst * 2), inc_d = (uint32_t)(kStep * a.dst * 2);
   const uint32_t so_q0 = (uint32_t)qfirst * (uint32_t)a.qst * 2, so_d0 = (uint32_t)qfirst * (uint32_t)a.dst * 2;
   int ld_it = 0, ld_h = kvh * a.G + g0, ld_qs = qfirst;
@@ -782,10 +782,12 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
   mfma_acc_drain();   // before the epilogue reads the AGPR accumulators
 
   // ---- epilogue: dK, dV (dV of a kv-head with a dead row is NaN) ---------------------
-  const bool dead = a.dead[b * a.Hk + kvh] != 0;
+  const auto& e = args_again<BwdArgs>();
+  const float scale = e.scale;
+  const bool dead = e.dead[b * e.Hk + kvh] != 0;
   const float nanv = __builtin_nanf("");
   lds_barrier();
-  if (a.split == 1 && (a.acc_mode == 0 || a.acc_mode == 3)) {
+  if (e.split == 1 && (e.acc_mode == 0 || e.acc_mode == 3)) {
     // stage [key][d] through LDS (wave-private rows), then coalesced 16-byte stores
     T* stg = (T*)smem + wave * 32 * OS;
     auto put = [&](const f32x16 (&acc)[NB], bool nan_out, T* dst, int64_t dstt) __attribute__((always_inline)) {
@@ -810,19 +812,19 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
 #pragma unroll
       for (int u = 0; u < NU; ++u) {
         const int idx = lane + u * 64, r = idx / CH, c = idx % CH;
-        if (kw0 + r < Tk) gstore16(dst + (int64_t)(kw0 + r) * dstt + c * 8, ov[u]);
+        if (kw0 + r < Tk && 8 * c < e.Dv) gstore16(dst + (int64_t)(kw0 + r) * dstt + c * 8, ov[u]);
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     };
-    if (a.acc_mode == 3) {
+    if (e.acc_mode == 3) {
       // last row range: the fp32 sums of the earlier ranges join (dK's scaled)
       if (key < Tk) {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
           for (int gi = 0; gi < 4; ++gi) {
-            const int64_t o = (((int64_t)b * Tk + key) * a.Hk + kvh) * D + nb * 32 + gi * 8 + hf * 4;
-            const f32x4 k4 = *(const f32x4*)(a.dk_accum + o), v4 = *(const f32x4*)(a.dv_accum + o);
+            const int64_t o = (((int64_t)b * Tk + key) * e.Hk + kvh) * D + nb * 32 + gi * 8 + hf * 4;
+            const f32x4 k4 = *(const f32x4*)(e.dk_accum + o), v4 = *(const f32x4*)(e.dv_accum + o);
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
               dkt[nb][gi * 4 + t] = dkt[nb][gi * 4 + t] * scale + k4[t];
@@ -834,30 +836,30 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) dkt[nb] *= scale;
     }
-    put(dkt, false, (T*)a.dk + b * a.dksb + kvh * a.dksh, a.dkst);
-    put(dvt, dead, (T*)a.dv + b * a.dvsb + kvh * a.dvsh, a.dvst);
+    put(dkt, false, (T*)e.dk + b * e.dksb + kvh * e.dksh, e.dkst);
+    put(dvt, dead, (T*)e.dv + b * e.dvsb + kvh * e.dvsh, e.dvst);
   } else {
     // fp32 slabs [split][B, Tk, Hk, D]: one per head-group split, summed in a
     // fixed order later; or, over row ranges, the running sums (acc_mode 1
     // writes them, 2 adds to them, in launch order)
-    const int64_t slab = (int64_t)sp * a.B * Tk * a.Hk * D;
-    const bool add = a.acc_mode == 2;
+    const int64_t slab = (int64_t)sp * e.B * Tk * e.Hk * D;
+    const bool add = e.acc_mode == 2;
     if (key < Tk) {
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
         for (int gi = 0; gi < 4; ++gi) {
           const int d = nb * 32 + gi * 8 + hf * 4;
-          const int64_t o = slab + (((int64_t)b * Tk + key) * a.Hk + kvh) * D + d;
+          const int64_t o = slab + (((int64_t)b * Tk + key) * e.Hk + kvh) * D + d;
           f32x4 k4, v4;
 #pragma unroll
           for (int t = 0; t < 4; ++t) { k4[t] = dkt[nb][gi * 4 + t] * scale; v4[t] = dead ? nanv : dvt[nb][gi * 4 + t]; }
           if (add) {
-            k4 += *(const f32x4*)(a.dk_accum + o);
-            v4 += *(const f32x4*)(a.dv_accum + o);
+            k4 += *(const f32x4*)(e.dk_accum + o);
+            v4 += *(const f32x4*)(e.dv_accum + o);
           }
-          *(f32x4*)(a.dk_accum + o) = k4;
-          *(f32x4*)(a.dv_accum + o) = v4;
+          *(f32x4*)(e.dk_accum + o) = k4;
+          *(f32x4*)(e.dv_accum + o) = v4;
         }
     }
   }

@@ -142,6 +142,18 @@ __device__ __forceinline__ void lds_write8(void* p, u32x2 v) {
 __device__ __forceinline__ u32x4 gload16(const void* p) {
   return *(const u32x4*)p;
 }
+// The same, or zeros where the memory holds no such columns (head dims below the
+// kernel's: Dv of D columns exist).
+__device__ __forceinline__ u32x4 gload16_if(bool ok, const void* p) {
+  return ok ? gload16(p) : u32x4{0, 0, 0, 0};
+}
+// x, or zeros (for columns that do not exist, after a load from one that does).
+__device__ __forceinline__ u32x4 zero_unless(bool ok, u32x4 x) { return ok ? x : u32x4{0, 0, 0, 0}; }
+// (Buffer records end after the Dv columns of the last row: rows may lie closer
+// together than the kernel's head dim is wide.)
+// Lane offset past every buffer's records (those stay below 2^31 bytes, and so
+// does any scalar offset added to it): the load returns zeros.
+constexpr uint32_t kNoRec = 0x80000000u;
 __device__ __forceinline__ void gstore16(void* p, u32x4 v) {
   *(u32x4*)p = v;
 }
@@ -179,6 +191,16 @@ __device__ __forceinline__ int chunk_swz(int r) {
 template <int W>
 __device__ __forceinline__ int tile_off(int r, int c) {
   return r * W + ((((c >> 3) ^ chunk_swz<W>(r))) << 3) + (c & 7);
+}
+
+// A kernel's (only) argument, read again from memory: what only the epilogue
+// needs then does not occupy scalar registers through the main loop (the
+// compiler loads a by-value argument's fields once, at the start).
+template <typename A>
+__device__ __forceinline__ const __attribute__((address_space(4))) A& args_again() {
+  auto p = (const __attribute__((address_space(4))) A*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *p;
 }
 
 // Maps a 1-D block index onto a logical work index so that consecutive

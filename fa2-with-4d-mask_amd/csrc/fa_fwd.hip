@@ -193,7 +193,7 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_kernel(const FwdArgs a) {
     const T* src = qp + (int64_t)min(qrow, Tq - 1) * a.qst + hf * 8;
 #pragma unroll
     for (int ds = 0; ds < DS; ++ds) {
-      u32x4 x = gload16(src + ds * 16);
+      u32x4 x = gload16_if(16 * ds < a.Dv, src + ds * 16);
       x ^= neg;
       qf[QLDS ? 0 : ds] = as_vec8<T>(x);
     }
@@ -280,8 +280,8 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_kernel(const FwdArgs a) {
 #pragma unroll
   for (int u = 0; u < IPW; ++u) {
     const int r = (wave * IPW + u) * RPI + lane / CH, c = lane % CH;
-    goff_k[u] = (uint32_t)(r * a.kst * 2) + (uint32_t)(c * 16);
-    goff_v[u] = (uint32_t)(r * a.vst * 2) + (uint32_t)(c * 16);
+    goff_k[u] = 8 * c < a.Dv ? (uint32_t)(r * a.kst * 2) + (uint32_t)(c * 16) : kNoRec;
+    goff_v[u] = 8 * c < a.Dv ? (uint32_t)(r * a.vst * 2) + (uint32_t)(c * 16) : kNoRec;
     soff_k[u] = opaque(lds0 + KOFF + r * ROWB + ((c ^ swz_k<D>(r)) * 16));
     soff_v[u] = opaque(lds0 + VOFF + r * ROWB + ((c ^ swz_v<D>(r)) * 16));
   }
@@ -294,7 +294,7 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_kernel(const FwdArgs a) {
     const T* tb = base;
     if (valid) {
       const int64_t rows = min(Tk - t * BN, BN);
-      nrec = (uint32_t)min_i64((rows - 1) * st * 2 + ROWB, 0xfffffff0);
+      nrec = (uint32_t)min_i64((rows - 1) * st * 2 + 2 * a.Dv, 0xfffffff0);
       tb = base + (int64_t)t * BN * st;
     }
     return __builtin_amdgcn_make_buffer_rsrc((void*)tb, (short)0, (int)nrec, 0x00020000);
@@ -309,11 +309,11 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_kernel(const FwdArgs a) {
   // issued in the softmax phase, whose instruction issue bounds the step.
   const int nt_full = min(nt, Tk / BN);   // tiles [0, nt_full) are whole
   auto nrec_of = [&](int64_t st) __attribute__((always_inline)) -> uint32_t {
-    return (uint32_t)min_i64((int64_t)(BN - 1) * st * 2 + ROWB, 0xfffffff0);
+    return (uint32_t)min_i64((int64_t)(BN - 1) * st * 2 + 2 * a.Dv, 0xfffffff0);
   };
   const uint32_t nrec_k = nrec_of(a.kst), nrec_v = nrec_of(a.vst);
-  const uint32_t tail_k = (uint32_t)((int64_t)(Tk - nt_full * BN - 1) * a.kst * 2 + ROWB);
-  const uint32_t tail_v = (uint32_t)((int64_t)(Tk - nt_full * BN - 1) * a.vst * 2 + ROWB);
+  const uint32_t tail_k = (uint32_t)((int64_t)(Tk - nt_full * BN - 1) * a.kst * 2 + 2 * a.Dv);
+  const uint32_t tail_v = (uint32_t)((int64_t)(Tk - nt_full * BN - 1) * a.vst * 2 + 2 * a.Dv);
   const T* kb_run = kp + (int64_t)2 * BN * a.kst;   // K(p+2) of the batch loaded next
   const T* vb_run = vp + (int64_t)BN * a.vst;       // V(p+1)
   auto rsrc_run = [&](const T* tb, uint32_t full, uint32_t tail, int t) __attribute__((always_inline)) {
@@ -398,7 +398,7 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_kernel(const FwdArgs a) {
     const T* src = qp + (int64_t)min(qrow, Tq - 1) * a.qst + hf * 8;
     u32x4 x[DS];
 #pragma unroll
-    for (int ds = 0; ds < DS; ++ds) x[ds] = gload16(src + ds * 16) ^ neg;
+    for (int ds = 0; ds < DS; ++ds) x[ds] = gload16_if(16 * ds < a.Dv, src + ds * 16) ^ neg;
 #pragma unroll
     for (int ds = 0; ds < DS; ++ds) lds_write16_at(qaddr ^ (uint32_t)(32 * ds), x[ds]);
   };
@@ -808,7 +808,7 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_kernel(const FwdArgs a) {
     const int idx = lane + u * 64;
     const int r = idx / CH, c = idx % CH;
     const int qr = q0w + r;
-    if (qr < Tq) gstore16(op + (int64_t)qr * a.ost + c * 8, ov[u]);
+    if (qr < Tq && 8 * c < a.Dv) gstore16(op + (int64_t)qr * a.ost + c * 8, ov[u]);
   }
   if (hf == 0 && qrow < Tq)
     a.lse[((int64_t)b * a.Hq + h) * Tq + qrow] = (l_tot > 0.f) ? m_run + log2_fast(l_tot) : kPosInf;
@@ -842,7 +842,7 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_kernel(const FwdArgs a) {
         const int idx = lane + u * 64;
         const int r = idx / CH, c = idx % CH;
         const int qr = q0w + r;
-        if (qr < Tq) gstore16(lp + (int64_t)qr * a.olst + c * 8, ov[u]);
+        if (qr < Tq && 8 * c < a.Dv) gstore16(lp + (int64_t)qr * a.olst + c * 8, ov[u]);
       }
     }
   }

@@ -109,6 +109,7 @@ struct FwdArgs {
   MaskLayout ml;
   void* olo;            // optional (mask or score): O's rounding residual, dtype, strided like O
   int64_t olsb, olst, olsh;
+  int Dv;               // columns of Q, K, V, O that exist (a multiple of 16, <= the kernel's head dim)
   int causal;           // keep j <= i (the few-rows kernel; the others are built for it)
   int mask4;            // mask rows 4-byte aligned: 32-bit loads allowed (few-rows kernel)
   // Key split: ns > 1 ranges of the key axis, one workgroup each.  Range i of
@@ -130,6 +131,7 @@ struct PreArgs {
   const void* olo;      // optional: O's rounding residual (Delta = sum dO (O + olo))
   int64_t olsb, olst, olsh;
   int B, Tq, Hq, Hk, G;
+  int Dv;               // columns that exist
   int is_causal;
   const char* mws;      // prepared mask (with a mask): tells rows without a kept key
   MaskLayout ml;
@@ -145,6 +147,7 @@ struct BwdArgs {
   int64_t dqsb, dqst, dqsh, dksb, dkst, dksh, dvsb, dvst, dvsh;
   int64_t msb, msh, msq, ssb, ssh, ssq;
   int B, Tq, Tk, Hq, Hk, G;
+  int Dv;               // columns of the 16-bit operands that exist (fp32 accumulators have all of D)
   int nkt;              // key tiles per (b, kv-head)
   // (batch, kv-head) units bk = b Hk + kv-head of this launch: bk0 ..
   // bk0 + nbk - 1 of the B Hk.  The dS-tile kernels run in slices of units

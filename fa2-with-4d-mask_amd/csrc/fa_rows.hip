@@ -89,7 +89,7 @@ __global__ __launch_bounds__(kRWaves * 64, D == 256 ? 1 : 2) void fwd_rows_kerne
     const uint32_t neg = a.qsign < 0.f ? 0x80008000u : 0u;
     const T* src = (const T*)a.q + b * a.qsb + h * a.qsh + (int64_t)tq * a.qst + hf * 8;
 #pragma unroll
-    for (int ds = 0; ds < DS; ++ds) qf[ds] = as_vec8<T>(gload16(src + ds * 16) ^ neg);
+    for (int ds = 0; ds < DS; ++ds) qf[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, src + ds * 16) ^ neg);
   }
   // (head dim 256: in AGPRs, which MFMA reads as well, to keep them out of the
   // 256 VGPRs of the loop)
@@ -115,7 +115,7 @@ __global__ __launch_bounds__(kRWaves * 64, D == 256 ? 1 : 2) void fwd_rows_kerne
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int idx = lane + u * 64;
-    goff_v[u] = (uint32_t)((idx / CH) * a.vst * 2) + (uint32_t)((idx % CH) * 16);
+    goff_v[u] = 8 * (idx % CH) < a.Dv ? (uint32_t)((idx / CH) * a.vst * 2) + (uint32_t)((idx % CH) * 16) : kNoRec;
   }
   const uint32_t goff_k = (uint32_t)(l32 * a.kst * 2) + (uint32_t)(hf * 16);
   // rows of tile t through a buffer from its first key; keys past Tk (and a
@@ -124,12 +124,12 @@ __global__ __launch_bounds__(kRWaves * 64, D == 256 ? 1 : 2) void fwd_rows_kerne
     const int rows = min(Tk - t * kRKeys, kRKeys);
     const bool ok = valid && rows > 0;
     return __builtin_amdgcn_make_buffer_rsrc((void*)(base + (ok ? (int64_t)t * kRKeys * st : 0)), (short)0,
-                                             ok ? (int)((int64_t)(rows - 1) * st * 2 + ROWB) : 0, 0x00020000);
+                                             ok ? (int)((int64_t)(rows - 1) * st * 2 + 2 * a.Dv) : 0, 0x00020000);
   };
   auto load_k = [&](int t, bool valid) __attribute__((always_inline)) {
     const auto rs = tile_rs(kp, a.kst, t, valid);
 #pragma unroll
-    for (int ds = 0; ds < DS; ++ds) kf[ds] = __builtin_amdgcn_raw_buffer_load_b128(rs, goff_k + 32 * ds, 0, 0);
+    for (int ds = 0; ds < DS; ++ds) kf[ds] = __builtin_amdgcn_raw_buffer_load_b128(rs, goff_k + 32 * ds, 16 * ds < a.Dv ? 0 : kNoRec, 0);
   };
   auto load_v = [&](int t, bool valid) __attribute__((always_inline)) {
     const auto rs = tile_rs(vp, a.vst, t, valid);
@@ -361,6 +361,7 @@ __global__ __launch_bounds__(kRWaves * 64, D == 256 ? 1 : 2) void fwd_rows_kerne
         a.part_ml[2 * pr + 1] = l;
       }
     } else {
+      if (8 * c >= a.Dv) continue;
       const float inv = 1.0f / l;
       x0 *= inv;
       x1 *= inv;
@@ -429,7 +430,7 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdArgs a) {
       x0[e] += __shfl_xor(x0[e], d);
       x1[e] += __shfl_xor(x1[e], d);
     }
-  if (grp != 0 || !mine) return;
+  if (grp != 0 || !mine || 8 * c >= a.Dv) return;
   const float inv = 1.0f / lt;
   x0 *= inv;
   x1 *= inv;

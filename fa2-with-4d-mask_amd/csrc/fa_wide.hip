@@ -116,7 +116,7 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdArgs a) {
     const uint32_t neg = a.qsign < 0.f ? 0x80008000u : 0u;
     const T* src = (const T*)a.q + b * a.qsb + h * a.qsh + (int64_t)qrow_c * a.qst + hf * 8;
 #pragma unroll
-    for (int ds = 0; ds < DS; ++ds) qf[ds] = as_vec8<T>(gload16(src + ds * 16) ^ neg);
+    for (int ds = 0; ds < DS; ++ds) qf[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, src + ds * 16) ^ neg);
   }
   // The fragment stays in AGPRs (MFMA reads its operands there too): 64
   // VGPRs that the pipelined loop needs, which the compiler otherwise shuffles
@@ -151,12 +151,12 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdArgs a) {
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int idx = tid + u * 256, r = idx / CH, c = idx % CH;
-    goff_k[u] = (uint32_t)(r * a.kst * 2 + c * 16);
-    goff_v[u] = (uint32_t)(r * a.vst * 2 + c * 16);
+    goff_k[u] = 8 * c < a.Dv ? (uint32_t)(r * a.kst * 2 + c * 16) : kNoRec;
+    goff_v[u] = 8 * c < a.Dv ? (uint32_t)(r * a.vst * 2 + c * 16) : kNoRec;
   }
   auto tile_rs = [&](const T* base, int64_t st, int t) __attribute__((always_inline)) {
     const int rows = min(Tk - t * BN, BN);
-    const uint32_t nrec = rows > 0 ? (uint32_t)((int64_t)(rows - 1) * st * 2 + 2 * D) : 0u;
+    const uint32_t nrec = rows > 0 ? (uint32_t)((int64_t)(rows - 1) * st * 2 + 2 * a.Dv) : 0u;
     return __builtin_amdgcn_make_buffer_rsrc((void*)(base + (rows > 0 ? (int64_t)t * BN * st : 0)), (short)0,
                                              (int)nrec, 0x00020000);
   };
@@ -385,7 +385,7 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdArgs a) {
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
       const int idx = lane + u * 64, r = idx / CH, c = idx % CH;
-      if (q0w + r < Tq) gstore16(op + (int64_t)(q0w + r) * st + c * 8, ov[u]);
+      if (q0w + r < Tq && 8 * c < a.Dv) gstore16(op + (int64_t)(q0w + r) * st + c * 8, ov[u]);
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   };
@@ -440,8 +440,8 @@ __global__ __launch_bounds__(256, 1) void kv_wide_kernel(const BwdArgs a) {
     const T* vp = (const T*)a.v + b * a.vsb + kvh * a.vsh + (int64_t)kc * a.vst + hf * 8;
 #pragma unroll
     for (int ds = 0; ds < DS; ++ds) {
-      kf[ds] = as_vec8<T>(gload16(kp + ds * 16));
-      if constexpr (DK) vf[ds] = as_vec8<T>(gload16(vp + ds * 16));
+      kf[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, kp + ds * 16));
+      if constexpr (DK) vf[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, vp + ds * 16));
     }
   }
   // The fragments stay in AGPRs (MFMA reads its operands there too); the
@@ -473,8 +473,9 @@ __global__ __launch_bounds__(256, 1) void kv_wide_kernel(const BwdArgs a) {
     for (int u = 0; u < U; ++u) {
       const int idx = tid + u * 256, r = idx / CH, c = idx % CH;
       const int qq = min(qs + r, Tq - 1);
-      qreg[u] = gload16(qh + (int64_t)qq * a.qst + c * 8);
-      dreg[u] = gload16(dh + (int64_t)qq * a.dst + c * 8);
+      const int cc = 8 * c < a.Dv ? c : 0;   // (columns that do not exist: zeroed when stored)
+      qreg[u] = gload16(qh + (int64_t)qq * a.qst + cc * 8);
+      dreg[u] = gload16(dh + (int64_t)qq * a.dst + cc * 8);
     }
     if (tid < 64) {
       const int qq = qs + l32;
@@ -488,8 +489,8 @@ __global__ __launch_bounds__(256, 1) void kv_wide_kernel(const BwdArgs a) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int idx = tid + u * 256, r = idx / CH, c = idx % CH;
-      lds_write16(qs_ + r * QS + c * 8, qreg[u]);
-      lds_write16(ds_ + r * QS + c * 8, dreg[u]);
+      lds_write16(qs_ + r * QS + c * 8, zero_unless(8 * c < a.Dv, qreg[u]));
+      lds_write16(ds_ + r * QS + c * 8, zero_unless(8 * c < a.Dv, dreg[u]));
     }
     if (tid < 64) lsd[buf][hf][l32] = lreg;
   };
@@ -634,7 +635,7 @@ __global__ __launch_bounds__(256, 1) void kv_wide_kernel(const BwdArgs a) {
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
       const int idx = lane + u * 64, r = idx / CH, c = idx % CH;
-      if (kw0 + r < Tk) gstore16(dst + (int64_t)(kw0 + r) * dstt + c * 8, ov[u]);
+      if (kw0 + r < Tk && 8 * c < a.Dv) gstore16(dst + (int64_t)(kw0 + r) * dstt + c * 8, ov[u]);
     }
   } else {
     // head-group split: fp32 slabs [split][B, Tk, Hk, D], summed in a fixed order later
@@ -721,8 +722,8 @@ __global__ __launch_bounds__(256, 1) void dq_wide_kernel(const BwdArgs a) {
     const T* ds_ = (const T*)a.dout + b * a.dsb + h * a.dsh + (int64_t)qrow_c * a.dst + hf * 8;
 #pragma unroll
     for (int ds = 0; ds < DS; ++ds) {
-      qf[ds] = as_vec8<T>(gload16(qs + ds * 16));
-      dof[ds] = as_vec8<T>(gload16(ds_ + ds * 16));
+      qf[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, qs + ds * 16));
+      dof[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, ds_ + ds * 16));
     }
   }
 #pragma unroll
@@ -756,12 +757,12 @@ __global__ __launch_bounds__(256, 1) void dq_wide_kernel(const BwdArgs a) {
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int r = 8 * wave + 2 * u + (lane >> 5), c = (lane & 31) ^ swz_w(r);
-    goff_k[u] = (uint32_t)(r * a.kst * 2 + c * 16);
-    goff_v[u] = (uint32_t)(r * a.vst * 2 + c * 16);
+    goff_k[u] = 8 * c < a.Dv ? (uint32_t)(r * a.kst * 2 + c * 16) : kNoRec;
+    goff_v[u] = 8 * c < a.Dv ? (uint32_t)(r * a.vst * 2 + c * 16) : kNoRec;
   }
   auto tile_rs = [&](const T* base, int64_t st, int t) __attribute__((always_inline)) {
     const int rows = min(Tk - t * BN, BN);
-    const uint32_t nrec = rows > 0 ? (uint32_t)((int64_t)(rows - 1) * st * 2 + 2 * D) : 0u;
+    const uint32_t nrec = rows > 0 ? (uint32_t)((int64_t)(rows - 1) * st * 2 + 2 * a.Dv) : 0u;
     return __builtin_amdgcn_make_buffer_rsrc((void*)(base + (rows > 0 ? (int64_t)t * BN * st : 0)), (short)0,
                                              (int)nrec, 0x00020000);
   };
@@ -958,7 +959,7 @@ __global__ __launch_bounds__(256, 1) void dq_wide_kernel(const BwdArgs a) {
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
     const int idx = lane + u * 64, r = idx / CH, c = idx % CH;
-    if (q0w + r < Tq) gstore16(dqp + (int64_t)(q0w + r) * a.dqst + c * 8, ov[u]);
+    if (q0w + r < Tq && 8 * c < a.Dv) gstore16(dqp + (int64_t)(q0w + r) * a.dqst + c * 8, ov[u]);
   }
 }
 

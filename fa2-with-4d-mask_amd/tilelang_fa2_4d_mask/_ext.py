@@ -53,6 +53,7 @@ class FaFwdParams(ctypes.Structure):
         ("o_lo_stride_b o_lo_stride_t o_lo_stride_h", _i64),
         ("workspace", _vp),
         ("workspace_bytes", _i64),
+        ("head_dim_in", _i32),
     )
 
 
@@ -79,6 +80,7 @@ class FaBwdParams(ctypes.Structure):
         ("ds_limit_bytes", _i64),
         ("mask_ws o_lo", _vp),
         ("o_lo_stride_b o_lo_stride_t o_lo_stride_h ds_tiles_elems", _i64),
+        ("head_dim_in", _i32),
     )
 
 

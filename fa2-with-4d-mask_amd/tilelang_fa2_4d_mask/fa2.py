@@ -25,9 +25,9 @@ What differs on purpose:
   skip tiles without a kept entry (the reference streams every tile's mask
   bytes, python/fa2.py:107-114, 261-280);
 * the kernels exist for head dims 64, 128 and 256 (the reference compiles
-  any D, python/fa2.py:33); other D up to 256 run zero-padded to the next of
-  those, which is exact (see ``kernel_head_dim``), at the price of padded
-  copies of the operands.  Head dim 256 has kernels of its own (128-row
+  any D, python/fa2.py:33); other D up to 256 run as the next of those with
+  zero columns after theirs, which is exact (see ``kernel_head_dim``): multiples
+  of 16 in place, the others in padded copies of the operands.  Head dim 256 has kernels of its own (128-row
   forward blocks, dK and dV in two launches, dQ recomputed in both backward
   modes: no dS workspace, no atomics).
 """
@@ -70,6 +70,13 @@ def kernel_head_dim(D: int) -> int:
         if D <= w:
             return w
     return D
+
+
+def _columns_in_place(D: int) -> bool:
+    """Whether the kernels take operands of head dim ``D`` as they lie in memory
+    (they read zeros for the missing columns of their own head dim, 16 at a
+    time); otherwise the operands are padded copies."""
+    return D % 16 == 0 and D <= KERNEL_HEAD_DIMS[-1]
 
 
 def _pad_head_dim(x: torch.Tensor, Dp: int) -> torch.Tensor:
@@ -226,15 +233,16 @@ def _forward_impl(q, k, v, Mask, Score, scale: float, is_causal: bool, residual:
     no mask, or neither the kernels nor, without ``residual``, a backward
     reads it) and, with ``residual`` and a mask or a score, O's rounding residual (else
     None: the backward then takes Delta from O as stored), plus the operands
-    as the kernels saw them (zero-padded to the kernel head dim, see
-    ``kernel_head_dim``)."""
+    as the kernels saw them (padded where the kernels do not take the
+    head dim in place)."""
     B, Tq, Hq, D_in = q.shape
     _, Tk, Hk, _ = k.shape
     D = kernel_head_dim(D_in)
-    q, k, v = (_pad_head_dim(x, D) for x in (q, k, v))
+    W = D_in if _columns_in_place(D_in) else D     # columns of the operands in memory
+    q, k, v = (_pad_head_dim(x, W) for x in (q, k, v))
     mask, mst = _kernel_side(Mask, torch.bool, B, Hq, Tq, Tk, "mask", q.device)
     score, sst = _kernel_side(Score, torch.float32, B, Hq, Tq, Tk, "score", q.device)
-    O = torch.empty((B, Tq, Hq, D), dtype=q.dtype, device=q.device)
+    O = torch.empty((B, Tq, Hq, W), dtype=q.dtype, device=q.device)
     LSE = torch.empty((B, Hq, Tq), dtype=torch.float32, device=q.device)
     O_lo = torch.empty_like(O) if residual and (mask is not None or score is not None) else None
     mask_ws = None
@@ -263,6 +271,7 @@ def _forward_impl(q, k, v, Mask, Score, scale: float, is_causal: bool, residual:
             p.mask_stride_b, p.mask_stride_h, p.mask_stride_q = mst
             p.score_stride_b, p.score_stride_h, p.score_stride_q = sst
             p.batch, p.seqlen_q, p.seqlen_k, p.heads_q, p.heads_k, p.head_dim = B, Tq, Tk, Hq, Hk, D
+            p.head_dim_in = W
             p.scale = scale
             p.is_causal = 1 if is_causal else 0
             p.dtype = _ext.dtype_code(q.dtype)
@@ -277,7 +286,7 @@ def _forward_impl(q, k, v, Mask, Score, scale: float, is_causal: bool, residual:
                 mask_ws = _prepare_mask(mask, mst, B, Hq, Tq, Tk, bool(is_causal), q.device)
                 p.mask_ws = mask_ws.data_ptr()
             _call(lib, "fa_fwd", p)
-    if D != D_in:
+    if W != D_in:
         O = O[..., :D_in].contiguous()
         O_lo = None if O_lo is None else O_lo[..., :D_in].contiguous()
     return O, LSE, mask_ws, O_lo, (q, k, v, mask, score, mst, sst)
@@ -289,21 +298,24 @@ def _backward_impl(do, q, k, v, O, LSE, mask, score, mask_ws, mst, sst, scale: f
     operands (Q, K, V as given or as the forward's kernels saw them); returns
     dQ, dK, dV in the input dtype, [B, T, H, D] contiguous with D that of dO.
     ``O_lo``: the forward's rounding residual of O (with a mask or a score),
-    added to O for Delta.  Head dims other than the kernels' run zero-padded
-    (``kernel_head_dim``)."""
+    added to O for Delta.  Head dims other than the kernels' run in place or
+    zero-padded (``_columns_in_place``)."""
     B, Tq, Hq, D_in = do.shape
     _, Tk, Hk, _ = k.shape
     D = kernel_head_dim(D_in)
-    q, k, v, O, do = (_pad_head_dim(x, D) for x in (q, k, v, O, do))
+    W = D_in if _columns_in_place(D_in) else D
+    if W < D and (Tq + 32) * 2 * max(abs(q.stride(1)), abs(do.stride(1)), W * Hq) >= ROW_SPAN_LIMIT // 2:
+        W = D                                      # past the kernels' reach without padding
+    q, k, v, O, do = (_pad_head_dim(x, W) for x in (q, k, v, O, do))
     if O_lo is not None:
-        O_lo = _pad_head_dim(O_lo, D)
+        O_lo = _pad_head_dim(O_lo, W)
     dev = q.device
     if mask is not None and mask_ws is None and B * Tq * Hq * Tk > 0:
         # the forward ran without a gradient in sight and read the mask bytes
         mask_ws = _prepare_mask(mask, mst, B, Hq, Tq, Tk, is_causal, dev)
-    dQ = torch.empty((B, Tq, Hq, D), dtype=q.dtype, device=dev)
-    dK = torch.empty((B, Tk, Hk, D), dtype=q.dtype, device=dev)
-    dV = torch.empty((B, Tk, Hk, D), dtype=q.dtype, device=dev)
+    dQ = torch.empty((B, Tq, Hq, W), dtype=q.dtype, device=dev)
+    dK = torch.empty((B, Tk, Hk, W), dtype=q.dtype, device=dev)
+    dV = torch.empty((B, Tk, Hk, W), dtype=q.dtype, device=dev)
     if B * Tq * Hq == 0 or Tk == 0:
         dQ.zero_()
         dK.zero_()
@@ -313,6 +325,7 @@ def _backward_impl(do, q, k, v, O, LSE, mask, score, mask_ws, mst, sst, scale: f
     q = _rows_reachable(q, Tq)
     p = _ext.FaBwdParams()
     p.batch, p.seqlen_q, p.seqlen_k, p.heads_q, p.heads_k, p.head_dim = B, Tq, Tk, Hq, Hk, D
+    p.head_dim_in = W
     p.scale = scale
     p.is_causal = 1 if is_causal else 0
     p.atomic_dq = 1 if use_atomic_backward else 0
@@ -363,7 +376,7 @@ def _backward_impl(do, q, k, v, O, LSE, mask, score, mask_ws, mst, sst, scale: f
     _call(lib, "fa_bwd_preprocess", p)
     _call(lib, "fa_bwd", p)
     _call(lib, "fa_bwd_finalize", p)
-    if D != D_in:
+    if W != D_in:
         dQ, dK, dV = (x[..., :D_in].contiguous() for x in (dQ, dK, dV))
     return dQ, dK, dV
 

@@ -82,6 +82,9 @@ typedef struct FaFwdParams {
                                     16-byte aligned (fa_fwd_plan gives the size); without it, or with
                                     less, the key axis is not split */
   int64_t workspace_bytes;       /* bytes at workspace */
+  int32_t head_dim_in;           /* columns of q, k, v, o (o_lo) that exist in memory, a multiple of 16 up to
+                                    head_dim; the problem is that of head_dim with zero columns after them
+                                    (not read, not written).  0: all head_dim */
 } FaFwdParams;
 
 /* How fa_fwd runs a problem, so the caller can provide the workspaces. */
@@ -136,6 +139,8 @@ typedef struct FaBwdParams {
   int64_t ds_tiles_elems;        /* 16-bit elements the caller allocated at ds_tiles; when ds_tiles is given
                                     it must be at least plan.ds_elems of this problem (which depends on
                                     whether a mask or a score is given), else FA_ERR_WORKSPACE */
+  int32_t head_dim_in;           /* as in FaFwdParams, for every 16-bit operand and output (the fp32
+                                    accumulators have all head_dim columns).  0: all head_dim */
 } FaBwdParams;
 
 /* Mask preparation: the bool mask of a problem turned into the workspace the
