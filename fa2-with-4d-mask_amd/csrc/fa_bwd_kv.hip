@@ -303,6 +303,18 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
   // the head part below 2^27.
   int pq[MASK ? 4 : 1] = {};
   const int psh = 32 - __builtin_clz((uint32_t)max(a.nq32 - 1, 1));
+  // The bases of a head (mask words, dS tiles, score) move only with the head:
+  // one wave per SIMD issues all of a step's instructions, and computing them
+  // per step (64-bit multiplies) cost the masked score instance 7 % (T 4096, Hq
+  // 16: 678 -> 632 us).
+  // Words of this wave's key block (the lanes' clamped keys share one) in a
+  // head's plane: scalar base, moved only with the head, + step 128 bytes + the
+  // lane's key.
+  const int mkb = __builtin_amdgcn_readfirstlane(kc >> 5);
+  auto mask_words = [&](int h) __attribute__((always_inline)) -> const char* {
+    return a.mws + a.ml.bitsT + mask_plane(a.ml, b, h) * a.ml.pbitsT + (int64_t)mkb * a.ml.wq * 128;
+  };
+  const char* m_head = MASK ? mask_words(ld_h) : nullptr;
   auto load_next = [&](auto Sc, auto Qc) __attribute__((always_inline)) {
     constexpr int S = decltype(Sc)::value;
     constexpr int Q = decltype(Qc)::value;
@@ -320,9 +332,9 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
         d_head = (const T*)a.dout + b * a.dsb + (int64_t)ld_h * a.dsh;
         l_head = a.lse + ((int64_t)b * a.Hq + ld_h) * Tq;
         e_head = a.delta + ((int64_t)b * a.Hq + ld_h) * Tq;
+        m_head = mask_words(ld_h);
       }
-      const uint32_t* bt = (const uint32_t*)(a.mws + a.ml.bitsT + mask_plane(a.ml, b, ld_h) * a.ml.pbitsT);
-      mq[Q] = bt[((int64_t)(kc >> 5) * a.ml.wq + (ld_qs >> 5)) * 32 + (kc & 31)];
+      mq[Q] = ((const uint32_t*)(m_head + (uint64_t)(uint32_t)(ld_qs >> 5) * 128))[kc & 31];
       pq[Q] = ((ld_h - h_first) << psh) | (ld_qs >> 5);
     }
     const auto rq = MASK ? rs_of(q_head, q_rec, live) : rq_c;
@@ -414,10 +426,19 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
   float sreg[SCORE ? 16 : 1];
   const uint32_t s_lane = SCORE ? (uint32_t)(((int64_t)4 * hf * a.ssq + kc) * 4) : 0u;
   const uint32_t s_row = (uint32_t)a.ssq * 4u;
+  // (records of a whole step and of the last, partial one; the head's scores
+  // move only with the head)
+  const uint32_t s_rec = SCORE ? (uint32_t)((int64_t)31 * a.ssq * 4 + (int64_t)Tk * 4) : 0u;
+  const uint32_t s_rec_t = SCORE ? (uint32_t)(((int64_t)((Tq - 1) & 31)) * a.ssq * 4 + (int64_t)Tk * 4) : 0u;
+  int s_h = it_h;
+  const float* s_head = SCORE ? a.score + b * a.ssb + (int64_t)s_h * a.ssh : nullptr;
   auto score_rs = [&](int h, int qs, bool live) __attribute__((always_inline)) {
-    const uint32_t nrec = live ? (uint32_t)(((int64_t)min(Tq - qs, 32) - 1) * a.ssq * 4 + (int64_t)Tk * 4) : 0u;
-    return __builtin_amdgcn_make_buffer_rsrc((void*)(a.score + b * a.ssb + (int64_t)h * a.ssh + (int64_t)qs * a.ssq),
-                                             (short)0, (int)nrec, 0x00020000);
+    if (SCORE && h != s_h) {
+      s_h = h;
+      s_head = a.score + b * a.ssb + (int64_t)s_h * a.ssh;
+    }
+    const uint32_t nrec = live ? (Tq - qs >= 32 ? s_rec : s_rec_t) : 0u;
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(s_head + (int64_t)qs * a.ssq), (short)0, (int)nrec, 0x00020000);
   };
   auto load_s = [&](const __amdgpu_buffer_rsrc_t& rs, int i) __attribute__((always_inline)) {
     sreg[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
@@ -440,7 +461,11 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
   // writes chunks 2 t + hf, i.e. one contiguous kilobyte of whole lines
   const uint32_t ds_vo = (uint32_t)(hf * 512 + l32 * 16);
   const int64_t ds_h0 = ((int64_t)b * a.Hq + it_h - ds_u0) * a.ds_plane + ds_row(qfirst >> 5, a.nk32, CAUSAL) - ds_r0 + kb32;
-  const uint16_t* it_ptr = (const uint16_t*)a.ds + ds_h0 * 1024 * NPART;
+  // (with a mask: tile of row step 0, whose steps are then added)
+  auto ds_head = [&](int h) __attribute__((always_inline)) -> const uint16_t* {
+    return (const uint16_t*)a.ds + (((int64_t)b * a.Hq + h - ds_u0) * a.ds_plane - ds_r0 + kb32) * 1024 * NPART;
+  };
+  const uint16_t* it_ptr = MASK ? ds_head(it_h) : (const uint16_t*)a.ds + ds_h0 * 1024 * NPART;
   auto ds_rs = __builtin_amdgcn_make_buffer_rsrc((void*)a.ds, (short)0, 0, 0x00020000);
   // descriptor of step j's tile, then advance (it_h, it_qs, it_tile) to step j+1
   auto next_step = [&](int j, uint32_t mreg, int pos_next) __attribute__((always_inline)) {
@@ -452,12 +477,15 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
       // block state the dQ kernel reads, without a scalar load
       const bool any = __builtin_amdgcn_ballot_w64(mreg != 0u) != 0;
       const bool ok = ds_on && j < n && (!CAUSAL || kb32 <= s) && any;
-      const int64_t tile = ((int64_t)b * a.Hq + it_h - ds_u0) * a.ds_plane + ds_row(s, a.nk32, CAUSAL) - ds_r0 + kb32;
-      ds_rs = __builtin_amdgcn_make_buffer_rsrc((void*)((uint16_t*)a.ds + tile * 1024 * NPART), (short)0,
+      ds_rs = __builtin_amdgcn_make_buffer_rsrc((void*)(it_ptr + ds_row(s, a.nk32, CAUSAL) * 1024 * NPART), (short)0,
                                                 ok ? 2048 * NPART : 0, 0x00020000);
       // step j+1 as the load cursor queued it (padding steps: row 0 of the
       // last head)
-      it_h = h_first + (pos_next >> psh);
+      const int h_new = h_first + (pos_next >> psh);
+      if (h_new != it_h) {   // the head's first tile moves only with the head
+        it_h = h_new;
+        it_ptr = ds_head(it_h);
+      }
       it_qs = kStep * (pos_next & ((1 << psh) - 1));
       return;
     }
