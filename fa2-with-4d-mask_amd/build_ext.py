@@ -1,5 +1,6 @@
 #!/usr/bin/env python3
-r"""Builds libfa2_4d_mask.so (gfx950) in-tree with hipcc.
+r"""Builds libfa2_4d_mask.so (gfx950) in-tree with hipcc, and the native eager
+host path _fa2_host.so (csrc/fa_host.cpp) with g++ against torch.
 
 Usage: python fa2-with-4d-mask_amd/build_ext.py [--jobs N] [--verbose] [--host-sanitize]
 
@@ -34,6 +35,7 @@ CSRC = HERE / "csrc"
 BUILD = HERE / "_build"
 LIBDIR = HERE / "tilelang_fa2_4d_mask" / "_lib"
 LIB = LIBDIR / "libfa2_4d_mask.so"
+HOST = LIBDIR / "_fa2_host.so"
 BUILD_SAN = HERE / "_build_hostsan"
 LIB_SAN = BUILD_SAN / "libfa2_4d_mask_hostsan.so"
 # Host-only sanitizers: each flag applies to the host compilation alone.
@@ -81,6 +83,26 @@ def _run(cmd: list[str], verbose: bool) -> None:
         print(out, flush=True)
 
 
+def build_host(verbose: bool = False) -> Path:
+    """The native eager host path (csrc/fa_host.cpp): a Python module against
+    torch's C++ API, host code only."""
+    import sysconfig
+
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    LIBDIR.mkdir(exist_ok=True)
+    tmp = HOST.with_suffix(".so.tmp")
+    inc = [root / "include", root / "include" / "torch" / "csrc" / "api" / "include",
+           Path(hipcc()).resolve().parent.parent / "include", sysconfig.get_paths()["include"]]
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{HERE.parent / 'include'}",
+          *(f"-isystem{i}" for i in inc), str(CSRC / "fa_host.cpp"), "-o", str(tmp), f"-L{root / 'lib'}",
+          "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"], verbose)
+    os.replace(tmp, HOST)
+    return HOST
+
+
 def build(jobs: int = 4, verbose: bool = False, host_sanitize: bool = False) -> Path:
     out_dir, lib = (BUILD_SAN, LIB_SAN) if host_sanitize else (BUILD, LIB)
     out_dir.mkdir(exist_ok=True)
@@ -93,8 +115,11 @@ def build(jobs: int = 4, verbose: bool = False, host_sanitize: bool = False) -> 
         _run([cc, *flags, *EXTRA_FLAGS.get(src, []), "-c", str(CSRC / src), "-o", str(o)], verbose)
         return o
 
-    with ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
+    with ThreadPoolExecutor(max_workers=max(1, jobs) + 1) as ex:
+        host = None if host_sanitize else ex.submit(build_host, verbose)
         objs = list(ex.map(obj, SOURCES))
+        if host is not None:
+            host.result()
     tmp = lib.with_suffix(".so.tmp")
     if host_sanitize:
         # host link against the shared sanitizer runtime (the device code is

@@ -15,6 +15,8 @@ handles and device pointers valid on both sides.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 from pathlib import Path
@@ -23,6 +25,7 @@ import torch  # noqa: F401  (must be loaded before the HIP library, see above)
 
 LIB_PATH = (Path(os.environ["FA2_4D_MASK_LIB"]) if os.environ.get("FA2_4D_MASK_LIB")
             else Path(__file__).resolve().parent / "_lib" / "libfa2_4d_mask.so")
+HOST_PATH = Path(__file__).resolve().parent / "_lib" / "_fa2_host.so"
 ABI_VERSION = 7
 
 FA_DTYPE_BF16 = 0
@@ -154,6 +157,33 @@ def load_library(path: os.PathLike | None = None) -> ctypes.CDLL:
         if path is None:
             _lib = lib
         return lib
+
+
+_host = None
+
+
+def load_host(general_backward, default_settings, ds_limit: int):
+    """Loads (once) and returns the native eager host path (csrc/fa_host.cpp),
+    bound to the loaded library; raises RuntimeError if it is absent."""
+    global _host
+    if _host is not None:
+        return _host
+    lib = load_library()
+    with _lock:
+        if _host is not None:
+            return _host
+        if not HOST_PATH.exists():
+            raise RuntimeError(f"{HOST_PATH} is not built: run `python fa2-with-4d-mask_amd/build_ext.py`")
+        loader = importlib.machinery.ExtensionFileLoader("_fa2_host", str(HOST_PATH))
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_fa2_host", loader))
+        loader.exec_module(mod)
+        if mod.ABI_VERSION != ABI_VERSION:
+            raise RuntimeError(f"{HOST_PATH}: ABI version {mod.ABI_VERSION} != {ABI_VERSION}, rebuild it")
+        fns = (lib.fa_fwd_plan, lib.fa_fwd, lib.fa_mask_plan, lib.fa_mask_prepare, lib.fa_bwd_plan,
+               lib.fa_bwd_preprocess, lib.fa_bwd, lib.fa_bwd_finalize)
+        mod.init([ctypes.cast(f, ctypes.c_void_p).value for f in fns], general_backward, default_settings, ds_limit)
+        _host = mod
+        return mod
 
 
 class FaError(RuntimeError):

@@ -39,6 +39,7 @@ import ctypes
 from typing import Optional
 
 import torch
+from torch.autograd import forward_ad
 from torch.autograd.function import once_differentiable
 
 from . import _ext
@@ -429,16 +430,57 @@ class _flash_attention_with_4d_mask(torch.autograd.Function):
         return dQ, dK, dV, None, None, None, None, None, None
 
 
+def _default_settings() -> bool:
+    """No setting that only the Python host path honours (read by the native
+    path's backward)."""
+    return _event_log is None and DS_LIMIT_BYTES == 0
+
+
+def _general_backward(dO, q, k, v, out, lse, mask, score, mask_ws, o_lo, scale, is_causal, use_atomic_backward, bhsd):
+    """dQ, dK, dV through the custom op, for a backward the native path does not
+    take (a dS limit, the event log, double backward, operands to copy); tensors
+    in the caller's layout."""
+    from . import ops  # noqa: F401
+
+    if bhsd:
+        dO, q, k, v, out = (x.transpose(1, 2) for x in (dO, q, k, v, out))
+    grads = torch.ops.tilelang_fa2_4d_mask.bwd(
+        dO, q, k, v, out, lse, mask, score, torch.empty((0,), dtype=torch.uint8, device=q.device) if mask_ws is None else mask_ws,
+        q.new_empty((0,)) if o_lo is None else o_lo, scale, is_causal, use_atomic_backward)
+    return tuple(g.transpose(1, 2) for g in grads) if bhsd else tuple(grads)
+
+
+def _plain_eager(*tensors) -> bool:
+    """Plain eager execution: nothing traces, transforms or intercepts the
+    operation (compile, fake tensors, dispatch / function modes, functorch,
+    forward-mode AD, jit tracing, the event log), and the tensors are ordinary
+    ones.  Only then may it bypass the registered custom ops."""
+    if torch.compiler.is_compiling() or _event_log is not None:
+        return False
+    c = torch._C
+    if (c._len_torch_dispatch_stack() or c._len_torch_function_stack() or c._are_functorch_transforms_active()
+            or c._get_tracing_state() is not None or forward_ad._current_level >= 0):
+        return False
+    return all(x is None or type(x) is torch.Tensor or type(x) is torch.nn.Parameter for x in tensors)
+
+
 def flash_attention_with_4d_mask(Q, K, V, Mask=None, Score=None, scale=None, is_causal=False,
                                  use_atomic_backward=True, bhsd_input=True):
     """``flash_attention_with_4d_mask(Q, K, V, Mask, Score, scale, is_causal,
     use_atomic_backward, bhsd_input)`` (python/fa2.py:558): same positional
     signature, defaults, checks and autograd behaviour as the reference's
-    ``Function.apply``; the work runs in the registered custom ops
-    ``tilelang_fa2_4d_mask::fwd`` / ``::bwd`` (ops.py), which torch.compile and
-    graph capture can trace."""
+    ``Function.apply``.  In plain eager execution the native host path runs it
+    (csrc/fa_host.cpp); whatever that does not take, and everything traced or
+    transformed, runs in the registered custom ops ``tilelang_fa2_4d_mask::fwd`` /
+    ``::bwd`` (ops.py), with the same launches."""
     from . import ops
 
+    if _plain_eager(Q, K, V, Mask, Score) and Q.is_cuda and Q.dim() == 4:
+        host = _ext.load_host(_general_backward, _default_settings, DS_LIMIT_DEFAULT)
+        O = host.attention(Q, K, V, Mask, Score, float(Q.shape[3] ** -0.5 if scale is None else scale),
+                           bool(is_causal), bool(use_atomic_backward), bool(bhsd_input))
+        if O is not None:
+            return O
     assert Q.dim() == 4 and K.dim() == 4 and V.dim() == 4
     q = Q.transpose(1, 2) if bhsd_input else Q
     k = K.transpose(1, 2) if bhsd_input else K
