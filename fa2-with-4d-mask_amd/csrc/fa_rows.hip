@@ -26,7 +26,7 @@
 // skipped before their K and V are loaded; likewise tiles whose scores are all
 // -inf (additive padding masks).
 //
-// Measured (bf16, Hq 32, Hk 8, D 128): one row against 16384 keys 15 us + 6 for
+// Measured (bf16, Hq 32, Hk 8, D 128): one row against 16384 keys 15 us + 5 for
 // the combine (67 MB of K and V; 330 us in fwd_kernel, 32 workgroups); a batch of
 // 16, 3001 keys, left padding up to half: 34 + 4 us (253 + 16 for the prepared
 // mask before), the live 150-190 MB at 4.5-5 TB/s.
@@ -381,20 +381,25 @@ __global__ __launch_bounds__(kRWaves * 64, D == 256 ? 1 : 2) void fwd_rows_kerne
 // ---------------------------------------------------------------------------
 // O and LSE from the partial results of a.ns key ranges
 // ---------------------------------------------------------------------------
-// LPR lanes per row: lane i < ns of them holds range i's maximum and sum; D / 8
-// lanes share the row's columns, and LPR / (D / 8) groups of those the ranges,
-// summed over the groups at the end (fixed order: deterministic).  Few ranges:
-// LPR = D / 8, several rows per wave, each lane reading all of its ranges; up to
-// 64 (decoding: few rows): a wave per row.  Bound by reading the partials, which
-// the launch before left in L2.
-template <typename T, int D, int LPR>
+// LPR lanes of a wave per row and NW waves: lane i < ns of them holds range i's
+// maximum and sum; D / 8 lanes share the row's columns, and the NW LPR / (D / 8)
+// groups of those the ranges, summed over the groups at the end (fixed order:
+// deterministic).  Few ranges: LPR = D / 8, several rows per wave, each lane
+// reading all of its ranges; up to 64 (decoding: few rows): a workgroup per row,
+// whose waves take a quarter of the ranges each (64 ranges of 32 rows: 4.6 us, 9.1
+// with a wave per row).  Bound by the latency and the
+// per-CU rate of reading the partials, which the launch before left in L2.
+template <typename T, int D, int LPR, int NW>
 __global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdArgs a) {
   using V8 = typename Vec8<T>::type;
-  constexpr int CH = D / 8, NG = LPR / CH, RPB = 256 / LPR;
-  const int lane = threadIdx.x % LPR, c = lane % CH, grp = lane / CH;
+  static_assert(NW == 1 || (NW == 4 && LPR == 64), "waves of one row");
+  constexpr int CH = D / 8, NG = NW * LPR / CH, RPB = 256 / (NW * LPR);
+  const int lane = threadIdx.x % LPR, c = lane % CH;
+  const int grp = (NW == 1 ? 0 : (int)(threadIdx.x / 64) * (LPR / CH)) + lane / CH;
   const int64_t rows = (int64_t)a.B * a.Hq * a.Tq;
-  const int64_t ri = min_i64((int64_t)blockIdx.x * RPB + threadIdx.x / LPR, rows - 1);
-  const bool mine = (int64_t)blockIdx.x * RPB + threadIdx.x / LPR < rows;
+  const int64_t rb = (int64_t)blockIdx.x * RPB + (NW == 1 ? threadIdx.x / LPR : 0);
+  const int64_t ri = min_i64(rb, rows - 1);
+  const bool mine = rb < rows;
   const int q = (int)(ri % a.Tq);
   const int64_t bh = ri / a.Tq;
   const int b = (int)(bh / a.Hq), h = (int)(bh - (int64_t)b * a.Hq);
@@ -411,9 +416,8 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdArgs a) {
 #pragma unroll
   for (int d = 1; d < LPR; d <<= 1) lt += __shfl_xor(lt, d);
   f32x4 x0 = f32x4{}, x1 = f32x4{};
-  // sixteen ranges' loads in flight per lane: with 64 ranges (decoding, few
-  // rows) the kernel is one load latency long
-#pragma unroll (LPR == 64 ? 16 : 8)
+  // (a lane's loads all in flight: one load latency)
+#pragma unroll 8
   for (int i = grp; i < (a.ns + NG - 1) / NG * NG; i += NG) {
     const float wi = __shfl(w, i, LPR);   // ranges past ns have weight 0
     const float* p = a.part_o + ((int64_t)min(i, a.ns - 1) * rows + ri) * D + c * 8;
@@ -430,6 +434,22 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdArgs a) {
       x0[e] += __shfl_xor(x0[e], d);
       x1[e] += __shfl_xor(x1[e], d);
     }
+  if constexpr (NW > 1) {   // lane c of each wave holds the wave's sum
+    __shared__ f32x4 part[NW][CH][2];
+    const int w = threadIdx.x / 64;
+    if (lane < CH) {
+      part[w][c][0] = x0;
+      part[w][c][1] = x1;
+    }
+    __syncthreads();
+    x0 = part[0][c][0];
+    x1 = part[0][c][1];
+#pragma unroll
+    for (int i = 1; i < NW; ++i) {
+      x0 += part[i][c][0];
+      x1 += part[i][c][1];
+    }
+  }
   if (grp != 0 || !mine || 8 * c >= a.Dv) return;
   const float inv = 1.0f / lt;
   x0 *= inv;
@@ -462,9 +482,9 @@ hipError_t launch_combine_t(const FwdArgs& a, hipStream_t s) {
   const int64_t rows = (int64_t)a.B * a.Hq * a.Tq;
   if (a.ns <= 8) {   // D / 8 >= 8 lanes per row
     constexpr int RPB = 256 / (D / 8);
-    hipLaunchKernelGGL((fwd_combine_kernel<T, D, D / 8>), dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((fwd_combine_kernel<T, D, D / 8, 1>), dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256), 0, s, a);
   } else {
-    hipLaunchKernelGGL((fwd_combine_kernel<T, D, 64>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((fwd_combine_kernel<T, D, 64, 4>), dim3((unsigned)rows), dim3(256), 0, s, a);
   }
   return hipGetLastError();
 }
