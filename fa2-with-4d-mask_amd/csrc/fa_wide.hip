@@ -400,7 +400,9 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdArgs a) {
 // ---------------------------------------------------------------------------
 // dV (WHICH 0) / dK (WHICH 1)
 // ---------------------------------------------------------------------------
-template <typename T, bool CAUSAL, bool MASK, bool SCORE, int WHICH>
+// FULL: all of the operands' columns exist; without it the staging zeroes the
+// missing ones (a select per staged register, 2 % of the kernel).
+template <typename T, bool CAUSAL, bool MASK, bool SCORE, int WHICH, bool FULL>
 __global__ __launch_bounds__(256, 1) void kv_wide_kernel(const BwdArgs a) {
   using V8 = typename Vec8<T>::type;
   constexpr int D = kWD, DS = D / 16, NB = D / 32, CH = D / 8;
@@ -440,8 +442,8 @@ __global__ __launch_bounds__(256, 1) void kv_wide_kernel(const BwdArgs a) {
     const T* vp = (const T*)a.v + b * a.vsb + kvh * a.vsh + (int64_t)kc * a.vst + hf * 8;
 #pragma unroll
     for (int ds = 0; ds < DS; ++ds) {
-      kf[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, kp + ds * 16));
-      if constexpr (DK) vf[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, vp + ds * 16));
+      kf[ds] = as_vec8<T>(gload16_if(FULL || 16 * ds < a.Dv, kp + ds * 16));
+      if constexpr (DK) vf[ds] = as_vec8<T>(gload16_if(FULL || 16 * ds < a.Dv, vp + ds * 16));
     }
   }
   // The fragments stay in AGPRs (MFMA reads its operands there too); the
@@ -473,7 +475,7 @@ __global__ __launch_bounds__(256, 1) void kv_wide_kernel(const BwdArgs a) {
     for (int u = 0; u < U; ++u) {
       const int idx = tid + u * 256, r = idx / CH, c = idx % CH;
       const int qq = min(qs + r, Tq - 1);
-      const int cc = 8 * c < a.Dv ? c : 0;   // (columns that do not exist: zeroed when stored)
+      const int cc = FULL || 8 * c < a.Dv ? c : 0;   // (columns that do not exist: zeroed when stored)
       qreg[u] = gload16(qh + (int64_t)qq * a.qst + cc * 8);
       dreg[u] = gload16(dh + (int64_t)qq * a.dst + cc * 8);
     }
@@ -489,8 +491,8 @@ __global__ __launch_bounds__(256, 1) void kv_wide_kernel(const BwdArgs a) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int idx = tid + u * 256, r = idx / CH, c = idx % CH;
-      lds_write16(qs_ + r * QS + c * 8, zero_unless(8 * c < a.Dv, qreg[u]));
-      lds_write16(ds_ + r * QS + c * 8, zero_unless(8 * c < a.Dv, dreg[u]));
+      lds_write16(qs_ + r * QS + c * 8, zero_unless(FULL || 8 * c < a.Dv, qreg[u]));
+      lds_write16(ds_ + r * QS + c * 8, zero_unless(FULL || 8 * c < a.Dv, dreg[u]));
     }
     if (tid < 64) lsd[buf][hf][l32] = lreg;
   };
@@ -635,7 +637,7 @@ __global__ __launch_bounds__(256, 1) void kv_wide_kernel(const BwdArgs a) {
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
       const int idx = lane + u * 64, r = idx / CH, c = idx % CH;
-      if (kw0 + r < Tk && 8 * c < a.Dv) gstore16(dst + (int64_t)(kw0 + r) * dstt + c * 8, ov[u]);
+      if (kw0 + r < Tk && (FULL || 8 * c < a.Dv)) gstore16(dst + (int64_t)(kw0 + r) * dstt + c * 8, ov[u]);
     }
   } else {
     // head-group split: fp32 slabs [split][B, Tk, Hk, D], summed in a fixed order later
@@ -985,21 +987,27 @@ hipError_t launch_fwd_w(const FwdArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <typename T, bool CAUSAL, int WHICH>
+template <typename T, bool CAUSAL, int WHICH, bool FULL>
 hipError_t launch_kv_w(const BwdArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)(a.nbk * a.nkt * a.split)), block(256);
   const bool m = a.mask != nullptr, sc = a.score != nullptr;
-  if (m && sc) hipLaunchKernelGGL((kv_wide_kernel<T, CAUSAL, true, true, WHICH>), grid, block, 0, s, a);
-  else if (m) hipLaunchKernelGGL((kv_wide_kernel<T, CAUSAL, true, false, WHICH>), grid, block, 0, s, a);
-  else if (sc) hipLaunchKernelGGL((kv_wide_kernel<T, CAUSAL, false, true, WHICH>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((kv_wide_kernel<T, CAUSAL, false, false, WHICH>), grid, block, 0, s, a);
+  if (m && sc) hipLaunchKernelGGL((kv_wide_kernel<T, CAUSAL, true, true, WHICH, FULL>), grid, block, 0, s, a);
+  else if (m) hipLaunchKernelGGL((kv_wide_kernel<T, CAUSAL, true, false, WHICH, FULL>), grid, block, 0, s, a);
+  else if (sc) hipLaunchKernelGGL((kv_wide_kernel<T, CAUSAL, false, true, WHICH, FULL>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((kv_wide_kernel<T, CAUSAL, false, false, WHICH, FULL>), grid, block, 0, s, a);
   return hipGetLastError();
 }
 
-template <typename T, bool CAUSAL>
+template <typename T, bool CAUSAL, bool FULL>
 hipError_t launch_kv_both(const BwdArgs& a, hipStream_t s) {
-  const hipError_t e = launch_kv_w<T, CAUSAL, 0>(a, s);
-  return e != hipSuccess ? e : launch_kv_w<T, CAUSAL, 1>(a, s);
+  const hipError_t e = launch_kv_w<T, CAUSAL, 0, FULL>(a, s);
+  return e != hipSuccess ? e : launch_kv_w<T, CAUSAL, 1, FULL>(a, s);
+}
+
+template <typename T>
+hipError_t launch_kv_c(const BwdArgs& a, bool causal, hipStream_t s) {
+  if (a.Dv == kWD) return causal ? launch_kv_both<T, true, true>(a, s) : launch_kv_both<T, false, true>(a, s);
+  return causal ? launch_kv_both<T, true, false>(a, s) : launch_kv_both<T, false, false>(a, s);
 }
 
 }  // namespace
@@ -1019,8 +1027,7 @@ hipError_t launch_fwd_wide(const FwdArgs& a, int dtype, bool causal, hipStream_t
 }
 
 hipError_t launch_bwd_kv_wide(const BwdArgs& a, int dtype, bool causal, hipStream_t s) {
-  if (dtype == 0) return causal ? launch_kv_both<bf16, true>(a, s) : launch_kv_both<bf16, false>(a, s);
-  return causal ? launch_kv_both<f16, true>(a, s) : launch_kv_both<f16, false>(a, s);
+  return dtype == 0 ? launch_kv_c<bf16>(a, causal, s) : launch_kv_c<f16>(a, causal, s);
 }
 
 }  // namespace fa
