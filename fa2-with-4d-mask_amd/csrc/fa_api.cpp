@@ -811,12 +811,13 @@ int fa_bwd_finalize(const FaBwdParams* p) {
       if ((st = launch_status(fa::launch_bwd_dq(a, p->head_dim, p->dtype, causal, s), "dq"))) return st;
     }
   }
+  fa::CvtJobs jobs{};
   if (dq_atomics(p)) {
     // dq_accum is head-major [B, Hq, Tq, D]
     const int64_t D = p->head_dim, Tq = p->seqlen_q, Hq = p->heads_q;
     fa::CvtArgs c{p->dq_accum, p->dq, p->dq_stride_b, p->dq_stride_t, p->dq_stride_h,
                   p->batch, p->seqlen_q, p->heads_q, columns(p), 1, 0, Hq * Tq * D, D, Tq * D};
-    if ((st = launch_status(fa::launch_convert(c, p->dtype, s), "dq convert"))) return st;
+    jobs.job[jobs.n++] = c;
   }
   if (split > 1) {
     // one slab per head-group part, summed in a fixed order
@@ -825,11 +826,12 @@ int fa_bwd_finalize(const FaBwdParams* p) {
     const int64_t D = p->head_dim, Tk = p->seqlen_k, Hk = p->heads_k;
     fa::CvtArgs ck{p->dk_accum, p->dk, p->dk_stride_b, p->dk_stride_t, p->dk_stride_h,
                    p->batch, p->seqlen_k, p->heads_k, columns(p), nslab, slab, Tk * Hk * D, Hk * D, D};
-    if ((st = launch_status(fa::launch_convert(ck, p->dtype, s), "dk convert"))) return st;
+    jobs.job[jobs.n++] = ck;
     fa::CvtArgs cv{p->dv_accum, p->dv, p->dv_stride_b, p->dv_stride_t, p->dv_stride_h,
                    p->batch, p->seqlen_k, p->heads_k, columns(p), nslab, slab, Tk * Hk * D, Hk * D, D};
-    if ((st = launch_status(fa::launch_convert(cv, p->dtype, s), "dv convert"))) return st;
+    jobs.job[jobs.n++] = cv;
   }
+  if (jobs.n) return launch_status(fa::launch_convert(jobs, p->dtype, s), "convert");
   return FA_OK;
 }
 

@@ -209,6 +209,13 @@ struct CvtArgs {
   int64_t split_stride;  // elements between slabs
   int64_t src_sb, src_st, src_sh;
 };
+// Up to three conversions (dQ, dK, dV) in one launch: conversion i takes the
+// workgroups [first[i], first[i + 1]).
+struct CvtJobs {
+  CvtArgs job[3];
+  int n;
+  unsigned first[4];
+};
 
 hipError_t launch_fwd(const FwdArgs& a, int D, int dtype, bool causal, hipStream_t s);
 // Few query rows (fa_rows.hip), a.ns key ranges; with a.ns > 1 followed by the combine.
@@ -222,7 +229,7 @@ hipError_t launch_bwd_dkdv2(const BwdArgs& a, int D, int dtype, bool causal, hip
 int dkdv2_block_keys();
 // dQ = scale * dS K from the dS tiles, 256 query rows per workgroup.
 hipError_t launch_bwd_dq_ds(const BwdArgs& a, int D, int dtype, bool causal, hipStream_t s);
-hipError_t launch_convert(const CvtArgs& a, int dtype, hipStream_t s);
+hipError_t launch_convert(CvtJobs& jobs, int dtype, hipStream_t s);   // fills jobs.first
 // Head dim 256 (fa_wide.hip): forward, 128 query rows per workgroup; dK and
 // dV in two launches over 128-key workgroups (grid nbk x nkt x split, dK/dV
 // written like the dK/dV kernel's: dtype, or fp32 slabs with a split).
