@@ -17,7 +17,7 @@
 #include "fa_kernels.h"
 
 namespace fa {
-int fwd_block_rows();
+int fwd_block_rows(int D, bool causal, bool mask, bool score);
 int dq_block_rows();
 // fa_noalloc.hip: the allocation-free backward's device scratch
 int64_t noalloc_scratch_bytes();
@@ -398,7 +398,8 @@ FwdPlan fwd_plan(const FaFwdParams* p) {
     const int64_t nt = (keys + fa::fwd_rows_keys() - 1) / fa::fwd_rows_keys();
     f.split = (int)std::max<int64_t>(1, std::min<int64_t>({2 * kCus / base, nt / 4, kMaxKeySplit}));
   } else if (p->head_dim <= 128) {
-    const int64_t base = (int64_t)p->batch * p->heads_q * ((p->seqlen_q + fa::fwd_block_rows() - 1) / fa::fwd_block_rows());
+    const int brows = fa::fwd_block_rows(p->head_dim, p->is_causal != 0, p->mask != nullptr, p->score != nullptr);
+    const int64_t base = (int64_t)p->batch * p->heads_q * ((p->seqlen_q + brows - 1) / brows);
     const int64_t nt = (keys + fa::kFwdKeys - 1) / fa::kFwdKeys;
     f.split = fwd_key_split(base, nt, rows, p->head_dim, p->mask || p->score);
   }
@@ -506,7 +507,7 @@ int fa_fwd(const FaFwdParams* p) {
   a.B = p->batch; a.Tq = p->seqlen_q; a.Tk = p->seqlen_k; a.Hq = p->heads_q; a.Hk = p->heads_k;
   a.G = p->heads_q / p->heads_k;
   a.Dv = columns(p);
-  const int fwd_rows = p->head_dim > 128 ? fa::fwd_wide_block_rows() : fa::fwd_block_rows();
+  const int fwd_rows = p->head_dim > 128 ? fa::fwd_wide_block_rows() : fa::fwd_block_rows(p->head_dim, p->is_causal != 0, p->mask != nullptr, p->score != nullptr);
   a.nqt = (p->seqlen_q + fwd_rows - 1) / fwd_rows;
   float sl2b;
   fill_scales(p->scale, &a.scale_log2, &a.qsign, &a.zero_scale, &sl2b);

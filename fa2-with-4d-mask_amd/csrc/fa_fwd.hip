@@ -2,7 +2,7 @@
 // 4D fp32 score.  Restates the maths of the reference's TileLang forward
 // (python/fa2.py:22-139) as a hand-written wave64 MFMA kernel.
 //
-// Work decomposition: one workgroup of 8 waves per (256 query rows, query
+// Work decomposition: one workgroup of 8 waves (fewer: fwd_waves) per (256 query rows, query
 // head, batch); each wave owns 32 query rows and walks the key axis in tiles
 // of 64 keys.  Per tile and wave:
 //   S^T[key, q] = K Q^T        32x32x16 MFMA, A = K rows from LDS, B = Q
@@ -55,10 +55,16 @@
 namespace fa {
 namespace {
 
-constexpr int kWaves = 8;               // two groups of four
-constexpr int kBM = kWaves * 32;        // query rows per workgroup
+// Waves per workgroup (32 query rows each).  Causal at head dim 64 without a
+// mask or score: 4, three workgroups per CU (168 registers, 48 KB of LDS), whose
+// lengths even out better over the CUs than those of one 256-row block per CU:
+// Hq 16, T 2048 39 -> 32 us, Hq 32 Hk 8 T 8192 310 -> 292, B1 T 256 10.2 -> 8.8 (B2
+// T 1000 Hq 32 23.7 -> 24.4).  Not causal, 8 share each tile among twice the rows:
+// MQA Tq 2048, Tk 16384 292 us against 300 with 4, Tq 512, Tk 8192 in key ranges 54
+// against 65.  With a mask the prepared lists are for 256 rows; at head dim 128
+// the two groups of the 8 alternate by design.
+constexpr int fwd_waves(int D, bool causal, bool mask, bool score) { return D == 64 && causal && !mask && !score ? 4 : 8; }
 constexpr int kBN = 64;                 // keys per tile
-constexpr int kThreads = kWaves * 64;
 constexpr float kFastSumMax = 256.0f;   // lane partial sum bound of the fast path
 
 template <int N> struct IC { static constexpr int value = N; };
@@ -106,9 +112,10 @@ __device__ __forceinline__ void lds_barrier() {
 // SPLIT: the key tiles of each block are cut into a.ns ranges, one workgroup
 // each, which leave fp32 partial results for fwd_combine_kernel (fa_rows.hip).
 template <typename T, int D, bool CAUSAL, bool MASK, bool SCORE, bool SPLIT>
-__global__ __launch_bounds__(kThreads, 1) void fwd_kernel(const FwdArgs a) {
+__global__ __launch_bounds__(fwd_waves(D, CAUSAL, MASK, SCORE) * 64, fwd_waves(D, CAUSAL, MASK, SCORE) == 4 ? 3 : 1) void fwd_kernel(const FwdArgs a) {
   using V8 = typename Vec8<T>::type;
-  constexpr int BM = kBM, BN = kBN;
+  constexpr int kWaves = fwd_waves(D, CAUSAL, MASK, SCORE), kThreads = kWaves * 64;
+  constexpr int BM = kWaves * 32, BN = kBN;
   constexpr int DS = D / 16;            // k-steps of S^T
   constexpr int NB = D / 32;            // 32-wide d blocks of O^T
   constexpr int CH = D / 8;             // 16-byte chunks per row
@@ -131,7 +138,7 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_kernel(const FwdArgs a) {
   static_assert(NBUF * TILEB <= 65536, "buffer + row offsets fit the 16-bit DS immediate");
   constexpr int OS = D + 8;             // epilogue O staging stride (elements)
   static_assert(kWaves * 32 * OS * 2 <= 2 * NBUF * TILEB, "O staging fits in the K/V buffers");
-  static_assert(BM == kFwdRows && BN == kFwdKeys, "prepared-mask lists are built for this tile shape");
+  static_assert(!MASK || (BM == kFwdRows && BN == kFwdKeys), "prepared-mask lists are built for this tile shape");
   // With a mask or a score, P enters O += P V as two 16-bit halves (the
   // rounded value and its rounding residual, one more MFMA each): rows that
   // see few keys (packed documents, steep position biases) would otherwise
@@ -850,8 +857,8 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_kernel(const FwdArgs a) {
 
 template <typename T, int D, bool CAUSAL, bool SPLIT>
 hipError_t launch_fwd_t(const FwdArgs& a, hipStream_t s) {
-  const dim3 grid((unsigned)(a.B * a.Hq * a.nqt * (SPLIT ? a.ns : 1))), block(kThreads);
   const bool m = a.mask != nullptr, sc = a.score != nullptr;
+  const dim3 grid((unsigned)(a.B * a.Hq * a.nqt * (SPLIT ? a.ns : 1))), block(fwd_waves(D, CAUSAL, m, sc) * 64);
   if (m && sc) hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, true, true, SPLIT>), grid, block, 0, s, a);
   else if (m) hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, true, false, SPLIT>), grid, block, 0, s, a);
   else if (sc) hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, false, true, SPLIT>), grid, block, 0, s, a);
@@ -867,7 +874,7 @@ hipError_t launch_fwd_d(const FwdArgs& a, bool causal, hipStream_t s) {
 
 }  // namespace
 
-int fwd_block_rows() { return kBM; }
+int fwd_block_rows(int D, bool causal, bool mask, bool score) { return fwd_waves(D, causal, mask, score) * 32; }
 
 hipError_t launch_fwd(const FwdArgs& a, int D, int dtype, bool causal, hipStream_t s) {
   if (dtype == 0) {
