@@ -307,6 +307,8 @@ std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& 
       v.scalar_type() != q.scalar_type())
     return std::nullopt;
   const bool grad = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad());
+  // a score alone that wants a gradient (it gets none): the custom op's node
+  if (!grad && at::GradMode::is_enabled() && score.defined() && score.requires_grad()) return std::nullopt;
   Forward f;
   {
     at::AutoDispatchBelowADInplaceOrView below;

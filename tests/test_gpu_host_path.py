@@ -126,6 +126,16 @@ def test_autograd_contract(cuda):
         g[0].sum().backward()
 
 
+def test_only_the_score_wants_a_gradient(cuda):
+    """It gets none, but the output takes part in autograd as through the custom op."""
+    q, k, v, do = _qkv(cuda, "bhsd")
+    score = torch.zeros((1, 1, 70, 90), device=cuda, requires_grad=True)
+    out = api.tilelang_flash_attention(q, k, v, score=score)
+    assert out.requires_grad
+    out.backward(do)
+    assert score.grad is None
+
+
 def test_settings_between_forward_and_backward(cuda, monkeypatch):
     """A dS limit or the event log set after the forward still rules its backward."""
     q, k, v, do = _qkv(cuda, "bhsd", Tq=300, Tk=300)
