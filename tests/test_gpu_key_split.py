@@ -136,6 +136,24 @@ def test_key_split(cuda, case):
     _check(2, *case, residual=True)
 
 
+# Causal at head dim 64: blocks of 128 rows (four waves) without a mask or score
+CAUSAL64 = [
+    (1, 4, 2, 64, 129, 129, torch.bfloat16, True, None, None, 0.125),     # second block of one row
+    (2, 12, 4, 64, 1999, 1999, torch.float16, True, None, None, 0.125),
+    (2, 64, 64, 64, 300, 70, torch.bfloat16, True, None, None, 0.125),    # rows past the keys, not split
+    (1, 2, 1, 64, 130, 1000, torch.bfloat16, True, None, None, -0.125),   # keys past the rows
+    (1, 2, 1, 64, 1100, 1100, torch.float16, True, None, None, 0.0),      # scale 0, split
+]
+
+
+@pytest.mark.parametrize("case", CAUSAL64, ids=lambda c: f"B{c[0]}H{c[1]}-{c[2]}D{c[3]}T{c[4]}-{c[5]}")
+def test_causal_head_dim_64(cuda, case):
+    B, Hq, Hk, D, Tq, Tk, dtype, causal, mask, score, scale = case
+    plan = _plan(B, Hq, Hk, D, Tq, Tk, causal, mask, score)
+    print("case", case, "ranges", plan.key_split, flush=True)
+    _check(4, *case)
+
+
 def test_backward_after_a_forward_that_read_the_mask_itself(cuda):
     """The fwd op without ``residual`` leaves no prepared mask where its kernels
     read the bytes; the bwd op then prepares it: same gradients as with it."""
