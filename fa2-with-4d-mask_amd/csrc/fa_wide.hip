@@ -1,6 +1,6 @@
 // Attention kernels for head dims above 128 on gfx950 (MI355X): instances at
-// head dim 256 (the host zero-pads other head dims in (128, 256], which is
-// exact).  The reference's TileLang kernels take the head dim as a
+// head dim 256 (other head dims in (128, 256] run here as zero columns after
+// theirs, which is exact).  The reference's TileLang kernels take the head dim as a
 // compile-time constant of any size (python/fa2.py:33); these restate their
 // maths (forward python/fa2.py:22-139, backward :181-302 / :305-426) with
 // tiles that operands of 512 bytes per row fit:
@@ -31,8 +31,8 @@
 //                    fragments (128) beside its working set would not fit the
 //                    register file at this head dim, so the dK launch
 //                    recomputes S.
-// dQ comes from the recompute kernel of fa_bwd.hip (dq_kernel), Delta and the
-// backward's LSE from its preprocess kernel.  Conventions as in the head-dim
+//   dq_wide_kernel   dQ recomputed, four waves per (128 query rows, head, batch).
+// Delta and the backward's LSE come from the preprocess kernel of fa_bwd.hip.  Conventions as in the head-dim
 // 64/128 kernels: masked entries get P = 0 by select after the exp; rows past
 // Tq carry LSE = +inf (P = 0); keys past Tk read key Tk-1 (finite) and are
 // masked; with a mask or a score, P and dS enter their products in several
@@ -248,7 +248,10 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdArgs a) {
   }
   if constexpr (SCORE) score_of(1, sc);
 
-  constexpr int AH = 3;   // LDS operand reads in flight per MFMA stream
+  // LDS operand reads in flight per MFMA stream.  B1 T4096 Hq16 Hk4 without a
+  // mask or score, causal / not: 3 216 / 344 us, 5 212 / 336, 6 214 / 325-336, 8
+  // 230 causal (registers); with the two-part P the registers hold 3.
+  constexpr int AH = PREC ? 3 : 5;
 #pragma nounroll
   for (int j = 0; j <= nt; ++j) {
     load_k(j + 2);

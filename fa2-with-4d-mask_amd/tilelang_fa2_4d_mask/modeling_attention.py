@@ -121,7 +121,7 @@ def tilelang_flash_attention(
             # computed on the entries the caller holds, then broadcast: a
             # [B, 1, Tq, Tk] mask stays one plane per sequence (expanded first,
             # the division wrote and the kernels read Hq of them: B4 T1000 Hq32
-            # D128 fp16 503 us a call, 146 now)
+            # D128 fp16 502 us a call, 127 now)
             additive = attention_mask.to(dtype=torch.float32)
             if attention_mask_is_scaled:
                 additive = additive / scale
