@@ -115,11 +115,23 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
   // K, V fragments (B operands of S = Q K^T, dP = dO V^T): lane holds
   // K[key][16 ds + 8 hf .. +7].  Keys past Tk read row Tk-1: their dK/dV
   // rows are never stored and nothing else depends on them.
+  // Missing columns (16 ds >= Dv) load the first ones and are zeroed in a branch
+  // of their own: a branch per load made each wave wait for its first load
+  // before it issued the others, and for all of them before the first Q / dO
+  // tile's (causal B2 T4096 Hq32 Hk8: 1.6-3.8 % over loads without a column
+  // test; now 0.3-0.6 %).
   V8 kf[DS], vf[DS];
 #pragma unroll
   for (int ds = 0; ds < DS; ++ds) {
-    kf[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, kp + (int64_t)kc * a.kst + ds * 16 + hf * 8));
-    vf[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, vp + (int64_t)kc * a.vst + ds * 16 + hf * 8));
+    const int col = (16 * ds < a.Dv ? ds * 16 : 0) + hf * 8;
+    kf[ds] = as_vec8<T>(gload16(kp + (int64_t)kc * a.kst + col));
+    vf[ds] = as_vec8<T>(gload16(vp + (int64_t)kc * a.vst + col));
+  }
+  if (a.Dv < D) {
+    asm volatile("" ::: "memory");   // (stays a branch: selects would wait for the loads here)
+#pragma unroll
+    for (int ds = 0; ds < DS; ++ds)
+      if (16 * ds >= a.Dv) kf[ds] = vf[ds] = as_vec8<T>(u32x4{0, 0, 0, 0});
   }
   // The fragments stay in AGPRs for the whole loop (MFMA reads its A and B
   // operands from AGPRs as well): 64 VGPRs freed, which the masked and score
