@@ -170,6 +170,22 @@ __device__ __forceinline__ float half_sum(float x) {
 }
 
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// The running maximum m (base 2, finite) raised to at least mc, in whole steps:
+// P then rounds the same whichever maximum was current, and exp2(m - raised) is an
+// exact power of two.  Across a gap that exp2 of has long underflowed (a tile of
+// large negative scores, -1e9 or the type's lowest value, came first) mc itself:
+// fp32's own steps at m, 128 at -1e9, are coarser, and m + ceil(mc - m) misses mc
+// by as much, so that P overflows or vanishes.  Up to 2^16 the sum is on mc's grid.
+__device__ __forceinline__ float raise_max(float m, float mc) {
+  const float gap = mc - m;
+  return gap > 65536.f ? mc : m + fmaxf(0.f, ceilf(gap));
+}
+// Whether a row's running maximum m = fl(s c) may lie so far (half an fp32 step)
+// from the product that fma(s, c, -m) keeps that exp2 of the difference is no
+// longer about 1 at the maximum: 2^64 at s c = -1e9, past every type at -1e30.
+// Such tiles take s - max(s) times c instead.  (Not for -inf: nothing kept yet.)
+__device__ __forceinline__ bool far_max(float m) { return fabsf(m) > 16777216.f && m > kNegInf; }
 __device__ __forceinline__ float log2_fast(float x) { return __builtin_amdgcn_logf(x); }
 
 __device__ __forceinline__ bool wave_any(bool p) {

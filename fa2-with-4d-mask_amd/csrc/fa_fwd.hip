@@ -497,6 +497,7 @@ __global__ __launch_bounds__(fwd_waves(D, CAUSAL, MASK, SCORE) * 64, fwd_waves(D
       }
   };
   float m_run = kNegInf, l_run = 0.f;
+  float m_fast = kPosInf;   // -m_run as the fast path of V(p) takes it (with a score)
 
   // ---- M(p): S(p) = K(p) Q^T and O += V(p-1)^T P(p-1) ---------------------------
   // S(p) is computed (and later discarded) also when p >= nt_w, and PV(p-1)
@@ -585,15 +586,19 @@ __global__ __launch_bounds__(fwd_waves(D, CAUSAL, MASK, SCORE) * 64, fwd_waves(D
     __builtin_amdgcn_s_setprio(0);
   };
 
-  // P = exp2(S c - m) packed into pk; returns the lane's partial row sum.
-  auto make_p = [&](float mneg) __attribute__((always_inline)) -> float {
+  // P = exp2(S c - m) packed into pk (SUB: exp2((S - sub) c - m)); returns the
+  // lane's partial row sum.
+  auto make_p = [&](float mneg, auto SUBc, float sub) __attribute__((always_inline)) -> float {
     float lsum = 0.f;
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
       const int kb = kk >> 1, c = kk & 1;
       float x[8];
 #pragma unroll
-      for (int t = 0; t < 8; ++t) x[t] = exp2_fast(fmaf(sacc[kb][8 * c + t], c2, mneg));
+      for (int t = 0; t < 8; ++t) {
+        const float s = sacc[kb][8 * c + t];
+        x[t] = exp2_fast(fmaf(decltype(SUBc)::value ? s - sub : s, c2, mneg));
+      }
       pk[kk] = pack8<T>(x[0], x[1], x[2], x[3], x[4], x[5], x[6], x[7]);
       if constexpr (PREC) {
         // residual of each rounded p (exact in fp32), itself rounded: pk + pkl
@@ -669,7 +674,7 @@ __global__ __launch_bounds__(fwd_waves(D, CAUSAL, MASK, SCORE) * 64, fwd_waves(D
     stage();
     // Fast path against the current m_run (+inf offset while m_run is -inf,
     // which makes the sum inf or NaN and forces the slow path).
-    float lsum = make_p(-m_run);
+    float lsum = make_p(SCORE ? m_fast : -m_run, IC<0>{}, 0.f);
     if (wave_any(!(lsum <= kFastSumMax))) {
       float mx = kNegInf;
 #pragma unroll
@@ -683,7 +688,7 @@ __global__ __launch_bounds__(fwd_waves(D, CAUSAL, MASK, SCORE) * 64, fwd_waves(D
       // rounds to the same 16-bit values whichever maximum was current (and
       // alpha below is an exact power of two)
       const float mc = mx * c2;
-      const float m_new = m_run == kNegInf ? mc : m_run + fmaxf(0.f, ceilf(mc - m_run));
+      const float m_new = m_run == kNegInf ? mc : raise_max(m_run, mc);
       const float alpha = (m_run == kNegInf) ? 0.f : exp2_fast(m_run - m_new);
       l_run *= alpha;
 #pragma unroll
@@ -691,7 +696,11 @@ __global__ __launch_bounds__(fwd_waves(D, CAUSAL, MASK, SCORE) * 64, fwd_waves(D
 #pragma unroll
         for (int e = 0; e < 16; ++e) oacc[nb][e] *= alpha;
       m_run = m_new;
-      lsum = make_p(m_run == kNegInf ? 0.f : -m_run);
+      const float mneg = m_run == kNegInf ? 0.f : -m_run;
+      m_fast = SCORE && far_max(m_run) ? kPosInf : -m_run;   // (far: every tile takes this path)
+      const bool far = SCORE && far_max(m_run) && mx > kNegInf;
+      if (SCORE && wave_any(far)) lsum = make_p(far ? mc - m_run : mneg, IC<1>{}, far ? mx : 0.f);
+      else lsum = make_p(mneg, IC<0>{}, 0.f);
     }
     l_run += lsum;
   };

@@ -263,16 +263,26 @@ __global__ __launch_bounds__(kRWaves * 64, D == 256 ? 1 : 2) void fwd_rows_kerne
       float mx = s[0];
 #pragma unroll
       for (int j = 1; j < 16; ++j) mx = fmaxf(mx, s[j]);
-      const float mc = half_max(mx) * c2;
+      mx = half_max(mx);
+      const float mc = mx * c2;
       if (wave_any(mc > m_run)) {
-        const float m_new = m_run == kNegInf ? mc : m_run + fmaxf(0.f, ceilf(mc - m_run));
+        const float m_new = m_run == kNegInf ? mc : raise_max(m_run, mc);
         const float alpha = m_run == kNegInf ? 0.f : exp2_fast(m_run - m_new);
         l_run *= alpha;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) oacc[nb] *= alpha;
         m_run = m_new;
       }
-      const float mneg = m_run == kNegInf ? 0.f : -m_run;
+      float mneg = m_run == kNegInf ? 0.f : -m_run;
+      if constexpr (SCORE) {
+        const bool far = far_max(m_run) && mx > kNegInf;
+        if (wave_any(far)) {
+          const float sub = far ? mx : 0.f;
+#pragma unroll
+          for (int j = 0; j < 16; ++j) s[j] -= sub;
+          if (far) mneg = mc - m_run;
+        }
+      }
       V8 pk[2], pkl[PREC ? 2 : 1];
 #pragma unroll
       for (int c = 0; c < 2; ++c) {

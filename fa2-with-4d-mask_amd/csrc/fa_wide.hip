@@ -304,7 +304,8 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdArgs a) {
     // The running maximum moves only when a row's maximum exceeds it by more
     // than kWLift (p stays below 2^kWLift meanwhile: O and l are fp32): the
     // rescale (O in AGPRs, read, scaled and written back) is rare.
-    const float mt = half_max(mx) * c2;   // the row's largest logit of tile j (scaled)
+    mx = half_max(mx);
+    const float mt = mx * c2;   // the row's largest logit of tile j (scaled)
     if (wave_any(mt > m_run + kWLift)) {
       const float m_new = fmaxf(m_run, mt);
       const float alpha = m_run == kNegInf ? 0.f : exp2_fast(m_run - m_new);
@@ -313,7 +314,16 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdArgs a) {
       for (int nb = 0; nb < NB; ++nb) oacc[nb] *= alpha;
       m_run = m_new;
     }
-    const float mneg = m_run == kNegInf ? 0.f : -m_run;
+    float mneg = m_run == kNegInf ? 0.f : -m_run;
+    if constexpr (SCORE) {
+      const bool far = far_max(m_run) && mx > kNegInf;
+      if (wave_any(far)) {
+        const float sub = far ? mx : 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s_cur[i] -= sub;
+        if (far) mneg = mt - m_run;
+      }
+    }
 
     // ---- block 2: S(j+1) || P(j) ---------------------------------------------------
     {
