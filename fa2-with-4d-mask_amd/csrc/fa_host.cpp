@@ -27,8 +27,8 @@ namespace {
 using at::Tensor;
 
 // Entry points of libfa2_4d_mask.so as the Python loader resolved them, and
-// the Python side: general_backward(...) and, of the module holding them, the
-// settings that send a backward there.
+// the Python side: general_backward(...), and whether a backward is a plain one
+// (nothing traces, transforms or intercepts it, and no setting sends it there).
 struct Api {
   int (*fwd_plan)(const FaFwdParams*, FaFwdPlan*);
   int (*fwd)(const FaFwdParams*);
@@ -41,8 +41,19 @@ struct Api {
 };
 Api g_api{};
 PyObject* g_general_backward = nullptr;   // callable, held for good
-PyObject* g_default_settings = nullptr;   // callable: no event log, no dS limit set
+PyObject* g_plain_backward = nullptr;     // callable
 int64_t g_ds_limit = 0;                   // the default limit
+
+// A dense device tensor that is its own memory: no batched, wrapped, negated,
+// all-zero or subclass tensor (batched gradients reach a backward as such), whose
+// data pointer is missing or means something else.
+bool plain(const Tensor& x) {
+  using K = c10::DispatchKey;
+  constexpr c10::DispatchKeySet wrapped({K::Python, K::Negative, K::Conjugate, K::ZeroTensor, K::Batched, K::FuncTorchBatched,
+                                         K::FuncTorchGradWrapper, K::Functionalize});
+  const c10::DispatchKeySet keys = x.key_set();
+  return keys.has(K::CUDA) && !keys.has_any(wrapped);
+}
 
 // The logical [B, T, H, D] view of a tensor given as [B, H, T, D] (bhsd) or
 // [B, T, H, D]: sizes, and strides with those of size-1 axes 0.
@@ -258,9 +269,9 @@ Gradients general_backward(const Tensor& dout, const Tensor& q, const Tensor& k,
   return {std::get<0>(r), std::get<1>(r), std::get<2>(r)};
 }
 
-bool default_settings() {
+bool plain_backward() {
   pybind11::gil_scoped_acquire gil;
-  return pybind11::handle(g_default_settings)().cast<bool>();
+  return pybind11::handle(g_plain_backward)().cast<bool>();
 }
 
 struct Attention : torch::autograd::Function<Attention> {
@@ -285,7 +296,7 @@ struct Attention : torch::autograd::Function<Attention> {
     const bool causal = flags & 1, atomic = flags >> 1 & 1, bhsd = flags >> 2 & 1;
     Gradients g;
     bool done = false;
-    if (!at::GradMode::is_enabled() && default_settings()) {
+    if (plain(grads[0]) && !at::GradMode::is_enabled() && plain_backward()) {
       at::AutoDispatchBelowADInplaceOrView below;
       done = ::backward(grads[0], s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7], s[8], scale, causal, atomic, bhsd, &g);
     }
@@ -306,6 +317,8 @@ std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& 
       (q.scalar_type() != at::kBFloat16 && q.scalar_type() != at::kHalf) || k.scalar_type() != q.scalar_type() ||
       v.scalar_type() != q.scalar_type())
     return std::nullopt;
+  if (!plain(q) || !plain(k) || !plain(v) || (mask.defined() && !plain(mask)) || (score.defined() && !plain(score)))
+    return std::nullopt;
   const bool grad = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad());
   // a score alone that wants a gradient (it gets none): the custom op's node
   if (!grad && at::GradMode::is_enabled() && score.defined() && score.requires_grad()) return std::nullopt;
@@ -320,13 +333,13 @@ std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& 
   return Attention::apply(q, k, v, f, scale, causal, atomic, bhsd);
 }
 
-void init(const std::vector<uintptr_t>& fn, pybind11::object general, pybind11::object defaults, int64_t ds_limit) {
+void init(const std::vector<uintptr_t>& fn, pybind11::object general, pybind11::object plain, int64_t ds_limit) {
   TORCH_CHECK(fn.size() == 8, "eight entry points expected");
   g_api = Api{(decltype(Api::fwd_plan))fn[0],     (decltype(Api::fwd))fn[1],  (decltype(Api::mask_plan))fn[2],
               (decltype(Api::mask_prepare))fn[3], (decltype(Api::bwd_plan))fn[4], (decltype(Api::bwd_preprocess))fn[5],
               (decltype(Api::bwd))fn[6],          (decltype(Api::bwd_finalize))fn[7]};
   g_general_backward = general.release().ptr();
-  g_default_settings = defaults.release().ptr();
+  g_plain_backward = plain.release().ptr();
   g_ds_limit = ds_limit;
 }
 

@@ -430,16 +430,10 @@ class _flash_attention_with_4d_mask(torch.autograd.Function):
         return dQ, dK, dV, None, None, None, None, None, None
 
 
-def _default_settings() -> bool:
-    """No setting that only the Python host path honours (read by the native
-    path's backward)."""
-    return _event_log is None and DS_LIMIT_BYTES == 0
-
-
 def _general_backward(dO, q, k, v, out, lse, mask, score, mask_ws, o_lo, scale, is_causal, use_atomic_backward, bhsd):
     """dQ, dK, dV through the custom op, for a backward the native path does not
-    take (a dS limit, the event log, double backward, operands to copy); tensors
-    in the caller's layout."""
+    take (a dS limit, the event log, double backward, batched gradients, dispatch
+    modes, operands to copy); tensors in the caller's layout."""
     from . import ops  # noqa: F401
 
     if bhsd:
@@ -464,6 +458,12 @@ def _plain_eager(*tensors) -> bool:
     return all(x is None or type(x) is torch.Tensor or type(x) is torch.nn.Parameter for x in tensors)
 
 
+def _plain_backward() -> bool:
+    """The same for a backward of the native path (whose node also looks at its
+    tensors), and no setting that only the Python host path honours."""
+    return DS_LIMIT_BYTES == 0 and _plain_eager()
+
+
 def flash_attention_with_4d_mask(Q, K, V, Mask=None, Score=None, scale=None, is_causal=False,
                                  use_atomic_backward=True, bhsd_input=True):
     """``flash_attention_with_4d_mask(Q, K, V, Mask, Score, scale, is_causal,
@@ -476,7 +476,7 @@ def flash_attention_with_4d_mask(Q, K, V, Mask=None, Score=None, scale=None, is_
     from . import ops
 
     if _plain_eager(Q, K, V, Mask, Score) and Q.is_cuda and Q.dim() == 4:
-        host = _ext.load_host(_general_backward, _default_settings, DS_LIMIT_DEFAULT)
+        host = _ext.load_host(_general_backward, _plain_backward, DS_LIMIT_DEFAULT)
         O = host.attention(Q, K, V, Mask, Score, float(Q.shape[3] ** -0.5 if scale is None else scale),
                            bool(is_causal), bool(use_atomic_backward), bool(bhsd_input))
         if O is not None:

@@ -198,3 +198,51 @@ def test_refusals(cuda, monkeypatch, bad):
                 F.flash_attention_with_4d_mask(q, k, v, mask)
             errors.append((type(e.value), str(e.value)))
     assert errors[0] == errors[1]
+
+
+def test_batched_output_gradients(cuda):
+    """A batch of output gradients in one backward (what a vectorised jacobian
+    does) is the loop over single ones."""
+    q, k, v, do = _qkv(cuda, "bhsd")
+    leaf = [x.detach().requires_grad_(True) for x in (q, k, v)]
+    G = torch.stack([do, 2 * do, torch.roll(do, 1, 2)])
+    out = api.tilelang_flash_attention(*leaf, use_atomic_backward=False)
+    got = torch.autograd.grad(out, leaf, G, is_grads_batched=True, retain_graph=True)
+    for i in range(3):
+        ref = torch.autograd.grad(out, leaf, G[i], retain_graph=True)
+        assert all(torch.equal(x[i], y) for x, y in zip(got, ref))
+
+
+def test_dispatch_mode_around_the_backward_sees_it(cuda):
+    """A dispatch mode entered after the forward sees the backward op, as it would
+    one from the general path."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    q, k, v, do = _qkv(cuda, "bhsd")
+    leaf = [x.detach().requires_grad_(True) for x in (q, k, v)]
+    ref = torch.autograd.grad(api.tilelang_flash_attention(*leaf, use_atomic_backward=False), leaf, do)
+    seen = []
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    out = api.tilelang_flash_attention(*leaf, use_atomic_backward=False)
+    with Mode():
+        got = torch.autograd.grad(out, leaf, do)
+    assert any("tilelang_fa2_4d_mask.bwd" in s for s in seen), seen
+    assert all(torch.equal(x, y) for x, y in zip(ref, got))
+
+
+def test_operands_that_are_not_their_memory(cuda, monkeypatch):
+    """Negated and all-zero tensors (what complex views and autograd make of them)."""
+    q, k, v, do = _qkv(cuda, "bhsd")
+    leaf = [x.detach().requires_grad_(True) for x in (q, k, v)]
+    _both(monkeypatch, lambda: _step(torch._neg_view(q), k, v, do, "bhsd"))
+    _both(monkeypatch, lambda: (api.tilelang_flash_attention(q, k, v, score=torch._neg_view(torch.ones((1, 1, 70, 90), device=cuda))),))
+    for g in (torch._neg_view(do), torch._efficientzerotensor(do.shape, dtype=do.dtype, device=cuda)):
+        out = api.tilelang_flash_attention(*leaf, use_atomic_backward=False)
+        got = torch.autograd.grad(out, leaf, g, retain_graph=True)
+        ref = torch.autograd.grad(out, leaf, (g + 0 * do).contiguous())
+        assert all(torch.equal(x, y) for x, y in zip(got, ref))
