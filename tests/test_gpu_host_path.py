@@ -246,3 +246,11 @@ def test_operands_that_are_not_their_memory(cuda, monkeypatch):
         got = torch.autograd.grad(out, leaf, g, retain_graph=True)
         ref = torch.autograd.grad(out, leaf, (g + 0 * do).contiguous())
         assert all(torch.equal(x, y) for x, y in zip(got, ref))
+
+
+def test_profiles_name_both_directions(cuda):
+    q, k, v, do = _qkv(cuda, "bhsd")
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        _step(q, k, v, do, "bhsd")
+    names = {e.key for e in prof.key_averages()}
+    assert {"tilelang_fa2_4d_mask::fwd", "tilelang_fa2_4d_mask::bwd"} <= names
