@@ -84,6 +84,17 @@ int dtype_code(const Tensor& q) { return q.scalar_type() == at::kBFloat16 ? FA_D
 
 void* stream_of(const Tensor& q) { return (void*)c10::hip::getCurrentHIPStream(q.device().index()).stream(); }
 
+// The mask of a forward's or backward's problem, to prepare.
+template <typename P> FaMaskParams mask_params(const P& p) {
+  FaMaskParams m{};
+  m.mask = p.mask;
+  m.mask_stride_b = p.mask_stride_b; m.mask_stride_h = p.mask_stride_h; m.mask_stride_q = p.mask_stride_q;
+  m.batch = p.batch; m.seqlen_q = p.seqlen_q; m.seqlen_k = p.seqlen_k; m.heads_q = p.heads_q;
+  m.is_causal = p.is_causal;
+  m.stream = p.stream;
+  return m;
+}
+
 struct Forward {
   Tensor out, lse, mask_ws, o_lo;   // out in the caller's layout; the last two undefined where not made
   Tensor mask, score;               // as given, undefined where not
@@ -147,12 +158,7 @@ bool forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& ma
     p.workspace_bytes = plan.workspace_bytes;
   }
   if (mask.defined() && (residual || plan.needs_mask_ws)) {
-    FaMaskParams m{};
-    m.mask = p.mask;
-    m.mask_stride_b = p.mask_stride_b; m.mask_stride_h = p.mask_stride_h; m.mask_stride_q = p.mask_stride_q;
-    m.batch = p.batch; m.seqlen_q = p.seqlen_q; m.seqlen_k = p.seqlen_k; m.heads_q = p.heads_q;
-    m.is_causal = p.is_causal;
-    m.stream = p.stream;
+    FaMaskParams m = mask_params(p);
     int64_t n = 0;
     if (g_api.mask_plan(&m, &n) != FA_OK) return false;
     f->mask_ws = at::empty({n}, bytes);
@@ -208,6 +214,11 @@ bool backward(const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor
     p.mask = (const uint8_t*)mask.const_data_ptr();
     p.mask_stride_b = side_stride(mask, 0); p.mask_stride_h = side_stride(mask, 1); p.mask_stride_q = side_stride(mask, 2);
     p.mask_ws = mask_ws.const_data_ptr();
+    // (prepared for the broadcast axes of the mask as it was: a hook that copies a
+    // broadcast mask gives back one with more planes than the workspace has)
+    const FaMaskParams m = mask_params(p);
+    int64_t n = 0;
+    if (g_api.mask_plan(&m, &n) != FA_OK || n != mask_ws.numel()) return false;
   }
   if (score.defined()) {
     p.score = (const float*)score.const_data_ptr();

@@ -106,7 +106,9 @@ def bwd(do: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: 
     vk = _fa2._kernel_operand(v) if B * Tq * Hq > 0 and Tk > 0 else v
     m, mst = _fa2._kernel_side(mask, torch.bool, B, Hq, Tq, Tk, "mask", q.device)
     s, sst = _fa2._kernel_side(score, torch.float32, B, Hq, Tq, Tk, "score", q.device)
-    ws = mask_ws if mask_ws.numel() else None
+    # the prepared mask, unless it is not one of this mask's layout (a hook that
+    # copies a broadcast mask gives back one with more planes than were prepared)
+    ws = mask_ws if mask_ws.numel() and mask_ws.numel() == _mask_ws_bytes(m, B, Hq, Tq, Tk, is_causal) else None
     lo = o_lo if o_lo.numel() else None
     dq, dk, dv = _fa2._backward_impl(do, qk, kk, vk, o, lse, m, s, ws, mst, sst, scale, is_causal,
                                      use_atomic_backward, lo)

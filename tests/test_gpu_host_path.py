@@ -254,3 +254,20 @@ def test_profiles_name_both_directions(cuda):
         _step(q, k, v, do, "bhsd")
     names = {e.key for e in prof.key_averages()}
     assert {"tilelang_fa2_4d_mask::fwd", "tilelang_fa2_4d_mask::bwd"} <= names
+
+
+@pytest.mark.parametrize("general", [False, True])
+def test_a_broadcast_mask_saved_on_the_host(cuda, monkeypatch, general):
+    """save_on_cpu gives back a copy with a plane per head of a mask that the
+    forward saw broadcast over them (and prepared as one plane)."""
+    q, k, v, do = _qkv(cuda, "bhsd")
+    leaf = [x.detach().requires_grad_(True) for x in (q, k, v)]
+    m = (torch.rand((2, 1, 70, 90), generator=torch.Generator().manual_seed(1)) < 0.8).to(cuda)
+    m[..., 0] = True
+    if general:
+        monkeypatch.setattr(F, "_plain_eager", lambda *t: False)
+    ref = torch.autograd.grad(api.tilelang_flash_attention(*leaf, mask=m, use_atomic_backward=False), leaf, do)
+    with torch.autograd.graph.save_on_cpu():
+        out = api.tilelang_flash_attention(*leaf, mask=m, use_atomic_backward=False)
+    got = torch.autograd.grad(out, leaf, do)
+    assert all(torch.equal(x, y) for x, y in zip(ref, got))
