@@ -176,17 +176,29 @@ struct Gradients {
 bool backward(const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& out, const Tensor& lse,
               const Tensor& mask, const Tensor& score, const Tensor& mask_ws, const Tensor& o_lo, double scale, bool causal,
               bool atomic, bool bhsd, Gradients* g) {
+  // saved tensors come back through hooks: as the forward saw them, or not here
+  const at::ScalarType dt = q.scalar_type();
+  auto as_saved = [&](const Tensor& x, at::ScalarType t) { return plain(x) && x.device() == q.device() && x.scalar_type() == t; };
+  if ((dt != at::kBFloat16 && dt != at::kHalf) || !as_saved(q, dt) || !as_saved(k, dt) || !as_saved(v, dt) ||
+      !as_saved(out, dt) || !as_saved(lse, at::kFloat) || (o_lo.defined() && !as_saved(o_lo, dt)) || q.dim() != 4 ||
+      k.dim() != 4 || !v.sizes().equals(k.sizes()) || !out.sizes().equals(q.sizes()) || !dout.sizes().equals(q.sizes()) ||
+      !lse.is_contiguous())
+    return false;
   const Operand oq = operand(q, bhsd), ok = operand(k, bhsd), ov = operand(v, bhsd), oo = operand(out, bhsd);
-  Tensor d = dout.scalar_type() == q.scalar_type() ? dout : dout.to(q.scalar_type());
+  if (ok.B != oq.B || ok.D != oq.D || ok.H == 0 || oq.H % ok.H != 0 || lse.numel() != oq.B * oq.H * oq.T ||
+      (o_lo.defined() && !o_lo.sizes().equals({oq.B, oq.T, oq.H, oq.D})))
+    return false;
+  Tensor d = dout.scalar_type() == dt ? dout : dout.to(dt);
   Operand od = operand(d, bhsd);
   if (!in_place(d, od)) {
     d = bhsd ? d.transpose(1, 2).contiguous().transpose(1, 2) : d.contiguous();
     od = operand(d, bhsd);
   }
-  // saved tensors come back through hooks: as the forward saw them, or not here
   if (!in_place(q, oq) || !in_place(k, ok) || !in_place(v, ov) || !in_place(out, oo) || !in_place(d, od)) return false;
-  if (mask.defined() && (!mask_ws.defined() || !side_ok(mask, at::kBool, q, oq.B, oq.H, oq.T, ok.T))) return false;
-  if (score.defined() && !side_ok(score, at::kFloat, q, oq.B, oq.H, oq.T, ok.T)) return false;
+  if (mask.defined() && (!mask_ws.defined() || !as_saved(mask_ws, at::kByte) || !mask_ws.is_contiguous() || !plain(mask) ||
+                         !side_ok(mask, at::kBool, q, oq.B, oq.H, oq.T, ok.T)))
+    return false;
+  if (score.defined() && (!plain(score) || !side_ok(score, at::kFloat, q, oq.B, oq.H, oq.T, ok.T))) return false;
   // rows the kernels reach with 32-bit byte offsets (fa2.py _rows_reachable);
   // half as far where columns are missing
   const int64_t far = (oq.T + 32) * 2 * std::max({std::abs(oq.st), std::abs(od.st), oq.D * oq.H});

@@ -100,7 +100,14 @@ def bwd(do: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: 
     """dQ, dK, dV ([B, T, H, D] contiguous, input dtype) of ``fwd``'s outputs."""
     B, Tq, Hq, D = q.shape
     Tk = k.shape[1]
-    # the operands exactly as the forward's kernels saw them
+    # the operands exactly as the forward's kernels saw them (saved tensors come
+    # back through hooks, which may have moved or converted them)
+    _fa2._check_qkv(q, k, v)
+    if any(x.device != q.device for x in (o, lse, mask_ws, o_lo)) or o.dtype != q.dtype or lse.dtype != torch.float32:
+        raise ValueError("o, lse, mask_ws and o_lo must be on the device of q, o and lse as fwd returned them")
+    if B * Tq * Hq > 0 and Tk > 0:
+        o, lse = _fa2._kernel_operand(o), lse.contiguous()
+        o_lo = _fa2._kernel_operand(o_lo) if o_lo.numel() else o_lo
     qk = _fa2._kernel_operand(q) if B * Tq * Hq > 0 and Tk > 0 else q
     kk = _fa2._kernel_operand(k) if B * Tq * Hq > 0 and Tk > 0 else k
     vk = _fa2._kernel_operand(v) if B * Tq * Hq > 0 and Tk > 0 else v

@@ -271,3 +271,31 @@ def test_a_broadcast_mask_saved_on_the_host(cuda, monkeypatch, general):
         out = api.tilelang_flash_attention(*leaf, mask=m, use_atomic_backward=False)
     got = torch.autograd.grad(out, leaf, do)
     assert all(torch.equal(x, y) for x, y in zip(ref, got))
+
+
+@pytest.mark.parametrize("side", [False, True])
+def test_saved_tensors_changed_by_hooks(cuda, side):
+    """Hooks that give saved tensors back laid out otherwise change nothing; those
+    that leave them in another type or on another device are refused."""
+    q, k, v, do = _qkv(cuda, "bhsd")
+    leaf = [x.detach().requires_grad_(True) for x in (q, k, v)]
+    kw = {}
+    if side:
+        g = torch.Generator().manual_seed(1)
+        m = torch.rand((2, 1, 70, 90), generator=g) < 0.8
+        m[..., 0] = True
+        kw = {"mask": m.to(cuda), "score": torch.randn((1, 4, 70, 90), generator=g).to(cuda)}
+
+    def grads(unpack):
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            out = api.tilelang_flash_attention(*leaf, use_atomic_backward=False, **kw)
+        return torch.autograd.grad(out, leaf, do)
+
+    ref = grads(lambda t: t)
+    for a, b in ((-1, -2), (0, 1)):
+        got = grads(lambda t: t.transpose(a, b).contiguous().transpose(a, b) if t.dim() > 1 else t)
+        assert all(torch.equal(x, y) for x, y in zip(ref, got))
+    for unpack in (lambda t: t.float(), lambda t: t.cpu(), lambda t: t.to(torch.float16) if t.is_floating_point() else t,
+                   lambda t: t.cpu() if t.dtype == torch.float32 else t):
+        with pytest.raises(ValueError):
+            grads(unpack)
