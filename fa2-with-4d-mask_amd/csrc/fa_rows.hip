@@ -23,8 +23,9 @@
 // A mask is read as the caller gives it, one byte per (row, key) -- these
 // launches read each byte once, so there is nothing to gain from the prepared
 // bit form and its three launches -- and tiles of which no row keeps a key are
-// skipped before their K and V are loaded; likewise tiles whose scores are all
-// -inf (additive padding masks).
+// skipped before their K and V are loaded.  (Not so tiles whose scores are all
+// -inf: their keys are kept, and a NaN or Inf in K or V reaches O as it does in
+// fa_fwd.hip.)
 //
 // Measured (bf16, Hq 32, Hk 8, D 128): one row against 16384 keys 15 us + 5 for
 // the combine (67 MB of K and V; 330 us in fwd_kernel, 32 workgroups); a batch of
@@ -187,33 +188,19 @@ __global__ __launch_bounds__(kRWaves * 64, D == 256 ? 1 : 2) void fwd_rows_kerne
   const int tr_col = ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
   char* vt = smem + wave * VT;
   uint32_t* keep = (uint32_t*)(smem + kRWaves * VT + wave * KEEPB);
-  // a tile of -inf scores adds nothing (with a scale <= 0 it is not -inf logits)
-  const bool skip_inf = SCORE && a.qsign > 0.f && !a.zero_scale;
 
   for (int ic = 0; ic < n_w; ic += kRScan) {
     // ---- live tiles among the next kRScan of this wave --------------------------
     const int cnt = min(kRScan, n_w - ic);
     uint32_t live = cnt == 32 ? ~0u : (1u << cnt) - 1u;
-    if (MASK || skip_inf) {
+    if constexpr (MASK) {
       live = 0;
 #pragma unroll 2
       for (int i = 0; i < cnt; ++i) {
         const int t = t_w + kRWaves * (ic + i);
-        uint32_t w = in_row(t * kRKeys);
-        if constexpr (MASK) w &= load_keep(t);
-        uint32_t any = w;
-        if constexpr (SCORE) {
-          if (skip_inf) {
-            f32x16 x;
-            load_score(t, x);
-            uint32_t fin = 0;
-#pragma unroll
-            for (int j = 0; j < 16; ++j) fin |= x[j] != kNegInf ? 1u << (8 * (j >> 2) + (j & 3)) : 0u;
-            any &= fin;
-          }
-        }
-        if constexpr (MASK) keep[i * 64 + lane] = w;
-        live |= wave_any(any != 0) ? 1u << i : 0u;
+        const uint32_t w = in_row(t * kRKeys) & load_keep(t);
+        keep[i * 64 + lane] = w;
+        live |= wave_any(w != 0) ? 1u << i : 0u;
       }
     }
     if (live == 0) continue;

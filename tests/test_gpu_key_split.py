@@ -168,3 +168,27 @@ def test_backward_after_a_forward_that_read_the_mask_itself(cuda):
     b = ops.bwd(do, q, k, v, O, L, m, None, ws1, lo, 0.125, False, False)
     for x, y in zip(a, b):
         assert torch.equal(x.isnan(), y.isnan()) and torch.equal(x.nan_to_num(), y.nan_to_num())
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("Tq", [1, 40, 200])
+@pytest.mark.parametrize("where", ["k", "v", "v_inf"])
+def test_non_finite_keys_under_infinite_scores(cuda, D, Tq, where):
+    """A score of -inf keeps its key: NaN in its K row, NaN or Inf in its V row
+    reach O (0 times them is NaN), whether or not other keys of its tile have
+    finite scores."""
+    q, k, v, _, _ = _inputs(5, 2, 4, 2, D, Tq, 300, torch.bfloat16, None, None)
+    s = torch.zeros((2, 1, Tq, 300))
+    s[0, ..., :200] = -math.inf         # whole tiles
+    s[1, ..., 100:105] = -math.inf
+    x = k if where == "k" else v
+    for b, h, j in ((0, 0, 70), (1, 1, 102)):
+        x[b, j, h] = math.inf if where == "v_inf" else math.nan
+    dv = [t.to(cuda) for t in (q, k, v)]
+    with torch.no_grad():
+        O = torch.ops.tilelang_fa2_4d_mask.fwd(*dv, None, s.to(cuda), 0.1, False, False, False)[0].cpu()
+    ref = E.eager_ref(*(t.transpose(1, 2).double() for t in (q, k, v)), None, s, scale=0.1, is_causal=False,
+                      compute_dtype=torch.float64).transpose(1, 2)
+    bad = torch.isnan(ref)
+    assert bad[0, :, :2].all() and bad[1, :, 2:].all() and not bad[0, :, 2:].any() and not bad[1, :, :2].any()
+    assert torch.equal(torch.isnan(O), bad)
