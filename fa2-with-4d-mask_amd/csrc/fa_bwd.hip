@@ -49,7 +49,8 @@ __device__ bool row_keeps_a_key(const PreArgs& a, int b, int h, int q) {
   return false;
 }
 
-template <typename T, int D>
+// FULL: all D columns exist (the loads then go out together).
+template <typename T, int D, bool FULL>
 __global__ __launch_bounds__(256) void preprocess_kernel(const PreArgs a) {
   constexpr int CH = D / 8;            // 16-byte chunks per row
   constexpr int CPT = CH / 4;          // chunks per thread (4 threads per row)
@@ -60,28 +61,21 @@ __global__ __launch_bounds__(256) void preprocess_kernel(const PreArgs a) {
   if (q < a.Tq) {
     const T* op = (const T*)a.o + b * a.osb + (int64_t)q * a.ost + h * a.osh;
     const T* dp = (const T*)a.dout + b * a.dsb + (int64_t)q * a.dst + h * a.dsh;
-    // sum over this thread's columns of x dO; the columns all exist (the loads
-    // then go out together) or not
-    auto dot = [&](const T* xp, bool all) __attribute__((always_inline)) {
+    // sum over this thread's columns of x dO
+    auto dot = [&](const T* xp) __attribute__((always_inline)) {
 #pragma unroll
       for (int u = 0; u < CPT; ++u) {
         const int c = part + 4 * u;
-        const auto xv = as_vec8<T>(all ? gload16(xp + c * 8) : gload16_if(8 * c < a.Dv, xp + c * 8));
-        const auto dv = as_vec8<T>(all ? gload16(dp + c * 8) : gload16_if(8 * c < a.Dv, dp + c * 8));
+        const auto xv = as_vec8<T>(gload16_if(FULL || 8 * c < a.Dv, xp + c * 8));
+        const auto dv = as_vec8<T>(gload16_if(FULL || 8 * c < a.Dv, dp + c * 8));
 #pragma unroll
         for (int t = 0; t < 8; ++t) acc = fmaf(to_f<T>(xv[t]), to_f<T>(dv[t]), acc);
       }
     };
     // O's rounding residual from the forward (mask or score): O to about 16
     // significant bits
-    const T* lp = (const T*)a.olo + b * a.olsb + (int64_t)q * a.olst + h * a.olsh;
-    if (a.Dv == D) {
-      dot(op, true);
-      if (a.olo) dot(lp, true);
-    } else {
-      dot(op, false);
-      if (a.olo) dot(lp, false);
-    }
+    dot(op);
+    if (a.olo) dot((const T*)a.olo + b * a.olsb + (int64_t)q * a.olst + h * a.olsh);
   }
   acc += __shfl_xor(acc, 1);
   acc += __shfl_xor(acc, 2);
@@ -120,11 +114,14 @@ constexpr int kDqBN = 64;    // keys per tile
 // dS work, which a lone wave issues in sequence (H: 2.53 -> 1.82 ms, causal
 // 1.47 -> 0.97).  The masked and score instances (P and dS in two parts)
 // keep one wave per SIMD: 256 registers would spill about a hundred.
-template <typename T, int D, bool CAUSAL, bool MASK, bool SCORE>
+// FULL: all D columns of the operands exist; otherwise Dv do (tested at run time,
+// the score instance took 6-10 % longer, the others 1-4 %: T 2048, Hq 16, Hk 4).
+template <typename T, int D, bool CAUSAL, bool MASK, bool SCORE, bool FULL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((MASK || SCORE) ? 1 : 2, (MASK || SCORE) ? 1 : 2)))
 void dq_kernel(const BwdArgs a) {
   using V8 = typename Vec8<T>::type;
   static_assert(D <= 128, "head dim 256 recomputes dQ in fa_wide.hip");
+  const int Dv = FULL ? D : a.Dv;
   constexpr int BM = kDqBM, BN = kDqBN;
   constexpr int NKB = BN / 32;   // 32-key blocks per tile
   constexpr int DS = D / 16, NB = D / 32, CH = D / 8;
@@ -163,10 +160,13 @@ void dq_kernel(const BwdArgs a) {
   V8 qf[DS], dof[DS];
   float lse_q = kPosInf, delta_q = 0.f;
   if (qrow < Tq) {
+    u32x4 xq[DS], xd[DS];
+    load_row(xq, qp + (int64_t)qrow * a.qst + hf * 8, Dv);
+    load_row(xd, dp + (int64_t)qrow * a.dst + hf * 8, Dv);
 #pragma unroll
     for (int ds = 0; ds < DS; ++ds) {
-      qf[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, qp + (int64_t)qrow * a.qst + ds * 16 + hf * 8));
-      dof[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, dp + (int64_t)qrow * a.dst + ds * 16 + hf * 8));
+      qf[ds] = as_vec8<T>(only_cols(xq[ds], ds, Dv));
+      dof[ds] = as_vec8<T>(only_cols(xd[ds], ds, Dv));
     }
     lse_q = a.lse[((int64_t)b * a.Hq + h) * Tq + qrow];
     delta_q = a.delta[((int64_t)b * a.Hq + h) * Tq + qrow];
@@ -212,7 +212,7 @@ void dq_kernel(const BwdArgs a) {
       const int idx = tid + u * 256;
       const int r = idx / CH, c = idx % CH;
       const int kk = min(k0 + r, Tk - 1);
-      const int cc = 8 * c < a.Dv ? c : 0;   // (columns that do not exist: zeroed when stored)
+      const int cc = FULL || 8 * c < Dv ? c : 0;   // (columns that do not exist: zeroed when stored)
       kreg[u] = gload16(kp + (int64_t)kk * a.kst + cc * 8);
       vreg[u] = gload16(vp + (int64_t)kk * a.vst + cc * 8);
     }
@@ -224,8 +224,8 @@ void dq_kernel(const BwdArgs a) {
     for (int u = 0; u < U; ++u) {
       const int idx = tid + u * 256;
       const int r = idx / CH, c = idx % CH;
-      lds_write16(ks + r * KS + c * 8, zero_unless(8 * c < a.Dv, kreg[u]));
-      lds_write16(vs + r * VS + c * 8, zero_unless(8 * c < a.Dv, vreg[u]));
+      lds_write16(ks + r * KS + c * 8, zero_unless(FULL || 8 * c < Dv, kreg[u]));
+      lds_write16(vs + r * VS + c * 8, zero_unless(FULL || 8 * c < Dv, vreg[u]));
     }
   };
 
@@ -341,7 +341,7 @@ void dq_kernel(const BwdArgs a) {
     const int idx = lane + u * 64;
     const int r = idx / CH, c = idx % CH;
     const int qr = q0w + r;
-    if (qr < Tq && 8 * c < a.Dv) gstore16(dqp + (int64_t)qr * a.dqst + c * 8, lds_read16(os + r * OS + c * 8));
+    if (qr < Tq && (FULL || 8 * c < Dv)) gstore16(dqp + (int64_t)qr * a.dqst + c * 8, lds_read16(os + r * OS + c * 8));
   }
 }
 
@@ -376,25 +376,36 @@ __global__ __launch_bounds__(256) void convert_kernel(const CvtJobs jobs) {
   }
 }
 
-template <typename T, int D, bool CAUSAL>
-hipError_t launch_dq_t(const BwdArgs& a, hipStream_t s) {
+template <typename T, int D, bool CAUSAL, bool FULL>
+hipError_t launch_dq_f(const BwdArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)(a.B * a.Hq * a.nqt)), block(256);
   const bool m = a.mask != nullptr, sc = a.score != nullptr;
-  if (m && sc) hipLaunchKernelGGL((dq_kernel<T, D, CAUSAL, true, true>), grid, block, 0, s, a);
-  else if (m) hipLaunchKernelGGL((dq_kernel<T, D, CAUSAL, true, false>), grid, block, 0, s, a);
-  else if (sc) hipLaunchKernelGGL((dq_kernel<T, D, CAUSAL, false, true>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((dq_kernel<T, D, CAUSAL, false, false>), grid, block, 0, s, a);
+  if (m && sc) hipLaunchKernelGGL((dq_kernel<T, D, CAUSAL, true, true, FULL>), grid, block, 0, s, a);
+  else if (m) hipLaunchKernelGGL((dq_kernel<T, D, CAUSAL, true, false, FULL>), grid, block, 0, s, a);
+  else if (sc) hipLaunchKernelGGL((dq_kernel<T, D, CAUSAL, false, true, FULL>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((dq_kernel<T, D, CAUSAL, false, false, FULL>), grid, block, 0, s, a);
+  return hipGetLastError();
+}
+
+template <typename T, int D, bool CAUSAL>
+hipError_t launch_dq_t(const BwdArgs& a, hipStream_t s) {
+  return a.Dv == D ? launch_dq_f<T, D, CAUSAL, true>(a, s) : launch_dq_f<T, D, CAUSAL, false>(a, s);
+}
+
+template <typename T, int D>
+hipError_t launch_pre_f(const PreArgs& a, hipStream_t s) {
+  const dim3 grid((unsigned)((a.Tq + 63) / 64), (unsigned)a.Hq, (unsigned)a.B), block(256);
+  if (a.Dv == D) hipLaunchKernelGGL((preprocess_kernel<T, D, true>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((preprocess_kernel<T, D, false>), grid, block, 0, s, a);
   return hipGetLastError();
 }
 
 template <typename T>
 hipError_t launch_pre_t(const PreArgs& a, int D, hipStream_t s) {
-  const dim3 grid((unsigned)((a.Tq + 63) / 64), (unsigned)a.Hq, (unsigned)a.B), block(256);
-  if (D == 128) hipLaunchKernelGGL((preprocess_kernel<T, 128>), grid, block, 0, s, a);
-  else if (D == 64) hipLaunchKernelGGL((preprocess_kernel<T, 64>), grid, block, 0, s, a);
-  else if (D == 256) hipLaunchKernelGGL((preprocess_kernel<T, 256>), grid, block, 0, s, a);
-  else return hipErrorInvalidValue;
-  return hipGetLastError();
+  if (D == 128) return launch_pre_f<T, 128>(a, s);
+  if (D == 64) return launch_pre_f<T, 64>(a, s);
+  if (D == 256) return launch_pre_f<T, 256>(a, s);
+  return hipErrorInvalidValue;
 }
 
 }  // namespace

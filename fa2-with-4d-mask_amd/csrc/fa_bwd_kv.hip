@@ -44,7 +44,9 @@ constexpr int kKvKeys = kKvWaves * 32;   // keys per workgroup
 constexpr int kStep = 32;                // query rows per step
 constexpr int kNBuf = 4;                 // LDS buffers of step tiles
 
-template <typename T, int D, bool CAUSAL, bool MASK, bool SCORE>
+// FULL: all D columns of the operands exist (a run-time test cost 0.3-0.6 % of the
+// causal launch at B2 T4096 Hq32 Hk8 D128: registers and the first loads' order).
+template <typename T, int D, bool CAUSAL, bool MASK, bool SCORE, bool FULL>
 __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void dkdv2_kernel(const BwdArgs a) {
   using V8 = typename Vec8<T>::type;
   constexpr int DS = D / 16, NB = D / 32, CH = D / 8, ROWB = 2 * D;
@@ -108,6 +110,7 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
   const int kc = min(key, Tk - 1);
   // scale == 0: every kept logit is 0, i.e. P = exp2(-LSE2): a zero multiplier
   const float c2 = a.zero_scale ? 0.f : a.scale_log2;
+  const int Dv = FULL ? D : a.Dv;
 
   const T* __restrict__ kp = (const T*)a.k + b * a.ksb + kvh * a.ksh;
   const T* __restrict__ vp = (const T*)a.v + b * a.vsb + kvh * a.vsh;
@@ -115,23 +118,16 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
   // K, V fragments (B operands of S = Q K^T, dP = dO V^T): lane holds
   // K[key][16 ds + 8 hf .. +7].  Keys past Tk read row Tk-1: their dK/dV
   // rows are never stored and nothing else depends on them.
-  // Missing columns (16 ds >= Dv) load the first ones and are zeroed in a branch
-  // of their own: a branch per load made each wave wait for its first load
-  // before it issued the others, and for all of them before the first Q / dO
-  // tile's (causal B2 T4096 Hq32 Hk8: 1.6-3.8 % over loads without a column
-  // test; now 0.3-0.6 %).
   V8 kf[DS], vf[DS];
+  {
+    u32x4 xk[DS], xv[DS];
+    load_row(xk, kp + (int64_t)kc * a.kst + hf * 8, Dv);
+    load_row(xv, vp + (int64_t)kc * a.vst + hf * 8, Dv);
 #pragma unroll
-  for (int ds = 0; ds < DS; ++ds) {
-    const int col = (16 * ds < a.Dv ? ds * 16 : 0) + hf * 8;
-    kf[ds] = as_vec8<T>(gload16(kp + (int64_t)kc * a.kst + col));
-    vf[ds] = as_vec8<T>(gload16(vp + (int64_t)kc * a.vst + col));
-  }
-  if (a.Dv < D) {
-    asm volatile("" ::: "memory");   // (stays a branch: selects would wait for the loads here)
-#pragma unroll
-    for (int ds = 0; ds < DS; ++ds)
-      if (16 * ds >= a.Dv) kf[ds] = vf[ds] = as_vec8<T>(u32x4{0, 0, 0, 0});
+    for (int ds = 0; ds < DS; ++ds) {
+      kf[ds] = as_vec8<T>(only_cols(xk[ds], ds, Dv));
+      vf[ds] = as_vec8<T>(only_cols(xv[ds], ds, Dv));
+    }
   }
   // The fragments stay in AGPRs for the whole loop (MFMA reads its A and B
   // operands from AGPRs as well): 64 VGPRs freed, which the masked and score
@@ -266,8 +262,8 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
 #pragma unroll
   for (int u = 0; u < UQ; ++u) {
     const int idx = tid + u * kKvWaves * 64, r = idx / CH, c = idx % CH;
-    gq[u] = 8 * c < a.Dv ? (uint32_t)(r * a.qst * 2 + c * 16) : kNoRec;
-    gd[u] = 8 * c < a.Dv ? (uint32_t)(r * a.dst * 2 + c * 16) : kNoRec;
+    gq[u] = FULL || 8 * c < Dv ? (uint32_t)(r * a.qst * 2 + c * 16) : kNoRec;
+    gd[u] = FULL || 8 * c < Dv ? (uint32_t)(r * a.dst * 2 + c * 16) : kNoRec;
     sw[u] = opaque(lds0 + r * ROWB + ((c ^ swz_q<D>(r)) * 16));
     if constexpr (SIX) sw2[u] = opaque(sw[u] + kHi);
   }
@@ -280,8 +276,8 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
   // range check includes, so rows past Tq read as zeros.  Padding steps use
   // descriptors without records.  State: next tile ld_it (head ld_h, first
   // row ld_qs), scalar byte offsets of that row in Q, dO and LSE/Delta.
-  const uint32_t q_rec = (uint32_t)((int64_t)(Tq - 1) * a.qst * 2 + 2 * a.Dv);
-  const uint32_t d_rec = (uint32_t)((int64_t)(Tq - 1) * a.dst * 2 + 2 * a.Dv);
+  const uint32_t q_rec = (uint32_t)((int64_t)(Tq - 1) * a.qst * 2 + 2 * Dv);
+  const uint32_t d_rec = (uint32_t)((int64_t)(Tq - 1) * a.dst * 2 + 2 * Dv);
   const uint32_t inc_q = (uint32_t)(kStep * a.qst * 2), inc_d = (uint32_t)(kStep * a.dst * 2);
   const uint32_t so_q0 = (uint32_t)qfirst * (uint32_t)a.qst * 2, so_d0 = (uint32_t)qfirst * (uint32_t)a.dst * 2;
   int ld_it = 0, ld_h = kvh * a.G + g0, ld_qs = qfirst;
@@ -852,7 +848,7 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
 #pragma unroll
       for (int u = 0; u < NU; ++u) {
         const int idx = lane + u * 64, r = idx / CH, c = idx % CH;
-        if (kw0 + r < Tk && 8 * c < e.Dv) gstore16(dst + (int64_t)(kw0 + r) * dstt + c * 8, ov[u]);
+        if (kw0 + r < Tk && (FULL || 8 * c < e.Dv)) gstore16(dst + (int64_t)(kw0 + r) * dstt + c * 8, ov[u]);
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     };
@@ -905,15 +901,20 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
   }
 }
 
-template <typename T, int D, bool CAUSAL>
-hipError_t launch_t(const BwdArgs& a, hipStream_t s) {
+template <typename T, int D, bool CAUSAL, bool FULL>
+hipError_t launch_f(const BwdArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)(a.nbk * a.nkt * a.nsp)), block(kKvWaves * 64);
   const bool m = a.mask != nullptr, sc = a.score != nullptr;
-  if (m && sc) hipLaunchKernelGGL((dkdv2_kernel<T, D, CAUSAL, true, true>), grid, block, 0, s, a);
-  else if (m) hipLaunchKernelGGL((dkdv2_kernel<T, D, CAUSAL, true, false>), grid, block, 0, s, a);
-  else if (sc) hipLaunchKernelGGL((dkdv2_kernel<T, D, CAUSAL, false, true>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((dkdv2_kernel<T, D, CAUSAL, false, false>), grid, block, 0, s, a);
+  if (m && sc) hipLaunchKernelGGL((dkdv2_kernel<T, D, CAUSAL, true, true, FULL>), grid, block, 0, s, a);
+  else if (m) hipLaunchKernelGGL((dkdv2_kernel<T, D, CAUSAL, true, false, FULL>), grid, block, 0, s, a);
+  else if (sc) hipLaunchKernelGGL((dkdv2_kernel<T, D, CAUSAL, false, true, FULL>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((dkdv2_kernel<T, D, CAUSAL, false, false, FULL>), grid, block, 0, s, a);
   return hipGetLastError();
+}
+
+template <typename T, int D, bool CAUSAL>
+hipError_t launch_t(const BwdArgs& a, hipStream_t s) {
+  return a.Dv == D ? launch_f<T, D, CAUSAL, true>(a, s) : launch_f<T, D, CAUSAL, false>(a, s);
 }
 
 }  // namespace

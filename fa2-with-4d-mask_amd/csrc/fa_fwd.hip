@@ -111,8 +111,12 @@ __device__ __forceinline__ void lds_barrier() {
 }
 // SPLIT: the key tiles of each block are cut into a.ns ranges, one workgroup
 // each, which leave fp32 partial results for fwd_combine_kernel (fa_rows.hip).
-template <typename T, int D, bool CAUSAL, bool MASK, bool SCORE, bool SPLIT>
+// FULL: all D columns of the operands exist; otherwise Dv do (a run-time value in the
+// prologue and the epilogue, 0.2-1.5 us of a launch: not where a short problem in one
+// range would notice).
+template <typename T, int D, bool CAUSAL, bool MASK, bool SCORE, bool SPLIT, bool FULL>
 __global__ __launch_bounds__(fwd_waves(D, CAUSAL, MASK, SCORE) * 64, fwd_waves(D, CAUSAL, MASK, SCORE) == 4 ? 3 : 1) void fwd_kernel(const FwdArgs a) {
+  const int Dv = FULL ? D : a.Dv;
   using V8 = typename Vec8<T>::type;
   constexpr int kWaves = fwd_waves(D, CAUSAL, MASK, SCORE), kThreads = kWaves * 64;
   constexpr int BM = kWaves * 32, BN = kBN;
@@ -198,12 +202,10 @@ __global__ __launch_bounds__(fwd_waves(D, CAUSAL, MASK, SCORE) * 64, fwd_waves(D
   auto load_q = [&]() __attribute__((always_inline)) {
     const uint32_t neg = a.qsign < 0.f ? 0x80008000u : 0u;
     const T* src = qp + (int64_t)min(qrow, Tq - 1) * a.qst + hf * 8;
+    u32x4 x[DS];
+    load_row(x, src, Dv);
 #pragma unroll
-    for (int ds = 0; ds < DS; ++ds) {
-      u32x4 x = gload16_if(16 * ds < a.Dv, src + ds * 16);
-      x ^= neg;
-      qf[QLDS ? 0 : ds] = as_vec8<T>(x);
-    }
+    for (int ds = 0; ds < DS; ++ds) qf[QLDS ? 0 : ds] = as_vec8<T>(only_cols(x[ds], ds, Dv, neg));
   };
 
   // Key tiles of the workgroup: 0 .. nt-1, or with a mask the live tiles of
@@ -287,8 +289,8 @@ __global__ __launch_bounds__(fwd_waves(D, CAUSAL, MASK, SCORE) * 64, fwd_waves(D
 #pragma unroll
   for (int u = 0; u < IPW; ++u) {
     const int r = (wave * IPW + u) * RPI + lane / CH, c = lane % CH;
-    goff_k[u] = 8 * c < a.Dv ? (uint32_t)(r * a.kst * 2) + (uint32_t)(c * 16) : kNoRec;
-    goff_v[u] = 8 * c < a.Dv ? (uint32_t)(r * a.vst * 2) + (uint32_t)(c * 16) : kNoRec;
+    goff_k[u] = 8 * c < Dv ? (uint32_t)(r * a.kst * 2) + (uint32_t)(c * 16) : kNoRec;
+    goff_v[u] = 8 * c < Dv ? (uint32_t)(r * a.vst * 2) + (uint32_t)(c * 16) : kNoRec;
     soff_k[u] = opaque(lds0 + KOFF + r * ROWB + ((c ^ swz_k<D>(r)) * 16));
     soff_v[u] = opaque(lds0 + VOFF + r * ROWB + ((c ^ swz_v<D>(r)) * 16));
   }
@@ -301,7 +303,7 @@ __global__ __launch_bounds__(fwd_waves(D, CAUSAL, MASK, SCORE) * 64, fwd_waves(D
     const T* tb = base;
     if (valid) {
       const int64_t rows = min(Tk - t * BN, BN);
-      nrec = (uint32_t)min_i64((rows - 1) * st * 2 + 2 * a.Dv, 0xfffffff0);
+      nrec = (uint32_t)min_i64((rows - 1) * st * 2 + 2 * Dv, 0xfffffff0);
       tb = base + (int64_t)t * BN * st;
     }
     return __builtin_amdgcn_make_buffer_rsrc((void*)tb, (short)0, (int)nrec, 0x00020000);
@@ -316,11 +318,11 @@ __global__ __launch_bounds__(fwd_waves(D, CAUSAL, MASK, SCORE) * 64, fwd_waves(D
   // issued in the softmax phase, whose instruction issue bounds the step.
   const int nt_full = min(nt, Tk / BN);   // tiles [0, nt_full) are whole
   auto nrec_of = [&](int64_t st) __attribute__((always_inline)) -> uint32_t {
-    return (uint32_t)min_i64((int64_t)(BN - 1) * st * 2 + 2 * a.Dv, 0xfffffff0);
+    return (uint32_t)min_i64((int64_t)(BN - 1) * st * 2 + 2 * Dv, 0xfffffff0);
   };
   const uint32_t nrec_k = nrec_of(a.kst), nrec_v = nrec_of(a.vst);
-  const uint32_t tail_k = (uint32_t)((int64_t)(Tk - nt_full * BN - 1) * a.kst * 2 + 2 * a.Dv);
-  const uint32_t tail_v = (uint32_t)((int64_t)(Tk - nt_full * BN - 1) * a.vst * 2 + 2 * a.Dv);
+  const uint32_t tail_k = (uint32_t)((int64_t)(Tk - nt_full * BN - 1) * a.kst * 2 + 2 * Dv);
+  const uint32_t tail_v = (uint32_t)((int64_t)(Tk - nt_full * BN - 1) * a.vst * 2 + 2 * Dv);
   const T* kb_run = kp + (int64_t)2 * BN * a.kst;   // K(p+2) of the batch loaded next
   const T* vb_run = vp + (int64_t)BN * a.vst;       // V(p+1)
   auto rsrc_run = [&](const T* tb, uint32_t full, uint32_t tail, int t) __attribute__((always_inline)) {
@@ -404,10 +406,9 @@ __global__ __launch_bounds__(fwd_waves(D, CAUSAL, MASK, SCORE) * 64, fwd_waves(D
     const uint32_t neg = a.qsign < 0.f ? 0x80008000u : 0u;
     const T* src = qp + (int64_t)min(qrow, Tq - 1) * a.qst + hf * 8;
     u32x4 x[DS];
+    load_row(x, src, Dv);
 #pragma unroll
-    for (int ds = 0; ds < DS; ++ds) x[ds] = gload16_if(16 * ds < a.Dv, src + ds * 16) ^ neg;
-#pragma unroll
-    for (int ds = 0; ds < DS; ++ds) lds_write16_at(qaddr ^ (uint32_t)(32 * ds), x[ds]);
+    for (int ds = 0; ds < DS; ++ds) lds_write16_at(qaddr ^ (uint32_t)(32 * ds), only_cols(x[ds], ds, Dv, neg));
   };
   // V (A operand of O^T via the transpose read): lane addresses key row
   // 32 (kk/2) + 16 (kk%2) + tr_row (+8), columns 32 nb + tr_col .. +3.
@@ -824,7 +825,7 @@ __global__ __launch_bounds__(fwd_waves(D, CAUSAL, MASK, SCORE) * 64, fwd_waves(D
     const int idx = lane + u * 64;
     const int r = idx / CH, c = idx % CH;
     const int qr = q0w + r;
-    if (qr < Tq && 8 * c < a.Dv) gstore16(op + (int64_t)qr * a.ost + c * 8, ov[u]);
+    if (qr < Tq && 8 * c < Dv) gstore16(op + (int64_t)qr * a.ost + c * 8, ov[u]);
   }
   if (hf == 0 && qrow < Tq)
     a.lse[((int64_t)b * a.Hq + h) * Tq + qrow] = (l_tot > 0.f) ? m_run + log2_fast(l_tot) : kPosInf;
@@ -858,27 +859,32 @@ __global__ __launch_bounds__(fwd_waves(D, CAUSAL, MASK, SCORE) * 64, fwd_waves(D
         const int idx = lane + u * 64;
         const int r = idx / CH, c = idx % CH;
         const int qr = q0w + r;
-        if (qr < Tq && 8 * c < a.Dv) gstore16(lp + (int64_t)qr * a.olst + c * 8, ov[u]);
+        if (qr < Tq && 8 * c < Dv) gstore16(lp + (int64_t)qr * a.olst + c * 8, ov[u]);
       }
     }
   }
 }
 
-template <typename T, int D, bool CAUSAL, bool SPLIT>
+template <typename T, int D, bool CAUSAL, bool SPLIT, bool FULL>
 hipError_t launch_fwd_t(const FwdArgs& a, hipStream_t s) {
   const bool m = a.mask != nullptr, sc = a.score != nullptr;
   const dim3 grid((unsigned)(a.B * a.Hq * a.nqt * (SPLIT ? a.ns : 1))), block(fwd_waves(D, CAUSAL, m, sc) * 64);
-  if (m && sc) hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, true, true, SPLIT>), grid, block, 0, s, a);
-  else if (m) hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, true, false, SPLIT>), grid, block, 0, s, a);
-  else if (sc) hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, false, true, SPLIT>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, false, false, SPLIT>), grid, block, 0, s, a);
+  if (m && sc) hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, true, true, SPLIT, FULL>), grid, block, 0, s, a);
+  else if (m) hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, true, false, SPLIT, FULL>), grid, block, 0, s, a);
+  else if (sc) hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, false, true, SPLIT, FULL>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, false, false, SPLIT, FULL>), grid, block, 0, s, a);
   return hipGetLastError();
+}
+
+template <typename T, int D, bool CAUSAL>
+hipError_t launch_fwd_c(const FwdArgs& a, hipStream_t s) {
+  if (a.ns > 1) return launch_fwd_t<T, D, CAUSAL, true, false>(a, s);
+  return a.Dv == D ? launch_fwd_t<T, D, CAUSAL, false, true>(a, s) : launch_fwd_t<T, D, CAUSAL, false, false>(a, s);
 }
 
 template <typename T, int D>
 hipError_t launch_fwd_d(const FwdArgs& a, bool causal, hipStream_t s) {
-  if (a.ns > 1) return causal ? launch_fwd_t<T, D, true, true>(a, s) : launch_fwd_t<T, D, false, true>(a, s);
-  return causal ? launch_fwd_t<T, D, true, false>(a, s) : launch_fwd_t<T, D, false, false>(a, s);
+  return causal ? launch_fwd_c<T, D, true>(a, s) : launch_fwd_c<T, D, false>(a, s);
 }
 
 }  // namespace

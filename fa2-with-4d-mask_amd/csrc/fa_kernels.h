@@ -102,6 +102,7 @@ struct FwdArgs {
   int64_t msb, msh, msq, ssb, ssh, ssq;
   int B, Tq, Tk, Hq, Hk, G;
   int nqt;              // query tiles per (b, h)
+  int Dv;               // columns of Q, K, V, O that exist (a multiple of 16, <= the kernel's head dim)
   float scale_log2;     // |scale| * log2(e)  (1 when zero_scale)
   float qsign;          // -1 folds a negative scale into Q and Score
   int zero_scale;       // scale == 0: every kept logit is 0
@@ -109,7 +110,6 @@ struct FwdArgs {
   MaskLayout ml;
   void* olo;            // optional (mask or score): O's rounding residual, dtype, strided like O
   int64_t olsb, olst, olsh;
-  int Dv;               // columns of Q, K, V, O that exist (a multiple of 16, <= the kernel's head dim)
   int causal;           // keep j <= i (the few-rows kernel; the others are built for it)
   int mask4;            // mask rows 4-byte aligned: 32-bit loads allowed (few-rows kernel)
   // Key split: ns > 1 ranges of the key axis, one workgroup each.  Range i of

@@ -89,8 +89,10 @@ __global__ __launch_bounds__(kRWaves * 64, D == 256 ? 1 : 2) void fwd_rows_kerne
   {
     const uint32_t neg = a.qsign < 0.f ? 0x80008000u : 0u;
     const T* src = (const T*)a.q + b * a.qsb + h * a.qsh + (int64_t)tq * a.qst + hf * 8;
+    u32x4 x[DS];
+    load_row(x, src, a.Dv);
 #pragma unroll
-    for (int ds = 0; ds < DS; ++ds) qf[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, src + ds * 16) ^ neg);
+    for (int ds = 0; ds < DS; ++ds) qf[ds] = as_vec8<T>(only_cols(x[ds], ds, a.Dv, neg));
   }
   // (head dim 256: in AGPRs, which MFMA reads as well, to keep them out of the
   // 256 VGPRs of the loop)

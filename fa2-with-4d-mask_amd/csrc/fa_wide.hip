@@ -63,10 +63,15 @@ __device__ __forceinline__ u32x2 pack4w(float x0, float x1, float x2, float x3) 
 // ---------------------------------------------------------------------------
 // forward
 // ---------------------------------------------------------------------------
-template <typename T, bool CAUSAL, bool MASK, bool SCORE>
+// FULL (all kernels here): all kWD columns of the operands exist; otherwise Dv do.
+// A constant there keeps the loops' schedule and register assignment those of
+// kernels without a column test (as a run-time value: causal dQ with a mask 180 ->
+// 193 us at B1 T2048 Hq16 Hk4, forward with a score 140 -> 143).
+template <typename T, bool CAUSAL, bool MASK, bool SCORE, bool FULL>
 __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdArgs a) {
   using V8 = typename Vec8<T>::type;
   constexpr int D = kWD, DS = D / 16, NB = D / 32, CH = D / 8;
+  const int Dv = FULL ? D : a.Dv;
   constexpr int BM = kWRows, BN = kWKeys;
   // padded row strides (elements): K rows are read 16 bytes per lane over 16
   // rows (a stride of 4 mod 64 banks), V by 4-row transpose reads of 64
@@ -115,8 +120,10 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdArgs a) {
   {
     const uint32_t neg = a.qsign < 0.f ? 0x80008000u : 0u;
     const T* src = (const T*)a.q + b * a.qsb + h * a.qsh + (int64_t)qrow_c * a.qst + hf * 8;
+    u32x4 x[DS];
+    load_row(x, src, Dv);
 #pragma unroll
-    for (int ds = 0; ds < DS; ++ds) qf[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, src + ds * 16) ^ neg);
+    for (int ds = 0; ds < DS; ++ds) qf[ds] = as_vec8<T>(only_cols(x[ds], ds, Dv, neg));
   }
   // The fragment stays in AGPRs (MFMA reads its operands there too): 64
   // VGPRs that the pipelined loop needs, which the compiler otherwise shuffles
@@ -151,12 +158,12 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdArgs a) {
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int idx = tid + u * 256, r = idx / CH, c = idx % CH;
-    goff_k[u] = 8 * c < a.Dv ? (uint32_t)(r * a.kst * 2 + c * 16) : kNoRec;
-    goff_v[u] = 8 * c < a.Dv ? (uint32_t)(r * a.vst * 2 + c * 16) : kNoRec;
+    goff_k[u] = 8 * c < Dv ? (uint32_t)(r * a.kst * 2 + c * 16) : kNoRec;
+    goff_v[u] = 8 * c < Dv ? (uint32_t)(r * a.vst * 2 + c * 16) : kNoRec;
   }
   auto tile_rs = [&](const T* base, int64_t st, int t) __attribute__((always_inline)) {
     const int rows = min(Tk - t * BN, BN);
-    const uint32_t nrec = rows > 0 ? (uint32_t)((int64_t)(rows - 1) * st * 2 + 2 * a.Dv) : 0u;
+    const uint32_t nrec = rows > 0 ? (uint32_t)((int64_t)(rows - 1) * st * 2 + 2 * Dv) : 0u;
     return __builtin_amdgcn_make_buffer_rsrc((void*)(base + (rows > 0 ? (int64_t)t * BN * st : 0)), (short)0,
                                              (int)nrec, 0x00020000);
   };
@@ -398,7 +405,7 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdArgs a) {
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
       const int idx = lane + u * 64, r = idx / CH, c = idx % CH;
-      if (q0w + r < Tq && 8 * c < a.Dv) gstore16(op + (int64_t)(q0w + r) * st + c * 8, ov[u]);
+      if (q0w + r < Tq && 8 * c < Dv) gstore16(op + (int64_t)(q0w + r) * st + c * 8, ov[u]);
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   };
@@ -413,8 +420,8 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdArgs a) {
 // ---------------------------------------------------------------------------
 // dV (WHICH 0) / dK (WHICH 1)
 // ---------------------------------------------------------------------------
-// FULL: all of the operands' columns exist; without it the staging zeroes the
-// missing ones (a select per staged register, 2 % of the kernel).
+// Without FULL the staging zeroes the missing columns (a select per staged
+// register, 2 % of the kernel).
 template <typename T, bool CAUSAL, bool MASK, bool SCORE, int WHICH, bool FULL>
 __global__ __launch_bounds__(256, 1) void kv_wide_kernel(const BwdArgs a) {
   using V8 = typename Vec8<T>::type;
@@ -688,10 +695,11 @@ __device__ __forceinline__ void lds_dma16(__amdgpu_buffer_rsrc_t rs, uint32_t ld
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (FA_LDS void*)(uintptr_t)lds_addr, 16, voff, 0, 0, 0);
 }
 
-template <typename T, bool CAUSAL, bool MASK, bool SCORE>
+template <typename T, bool CAUSAL, bool MASK, bool SCORE, bool FULL>
 __global__ __launch_bounds__(256, 1) void dq_wide_kernel(const BwdArgs a) {
   using V8 = typename Vec8<T>::type;
   constexpr int D = kWD, DS = D / 16, NB = D / 32, CH = D / 8;
+  const int Dv = FULL ? D : a.Dv;
   constexpr int BM = kWDqRows, BN = kWKeys;
   constexpr int TILEB = BN * D * 2;       // bytes of one K or V tile (32 rows of 512 bytes)
   // K tile t is read as rows by S(t) in iteration t-1 and transposed by
@@ -735,10 +743,13 @@ __global__ __launch_bounds__(256, 1) void dq_wide_kernel(const BwdArgs a) {
   {
     const T* qs = (const T*)a.q + b * a.qsb + h * a.qsh + (int64_t)qrow_c * a.qst + hf * 8;
     const T* ds_ = (const T*)a.dout + b * a.dsb + h * a.dsh + (int64_t)qrow_c * a.dst + hf * 8;
+    u32x4 xq[DS], xd[DS];
+    load_row(xq, qs, Dv);
+    load_row(xd, ds_, Dv);
 #pragma unroll
     for (int ds = 0; ds < DS; ++ds) {
-      qf[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, qs + ds * 16));
-      dof[ds] = as_vec8<T>(gload16_if(16 * ds < a.Dv, ds_ + ds * 16));
+      qf[ds] = as_vec8<T>(only_cols(xq[ds], ds, Dv));
+      dof[ds] = as_vec8<T>(only_cols(xd[ds], ds, Dv));
     }
   }
 #pragma unroll
@@ -772,12 +783,12 @@ __global__ __launch_bounds__(256, 1) void dq_wide_kernel(const BwdArgs a) {
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int r = 8 * wave + 2 * u + (lane >> 5), c = (lane & 31) ^ swz_w(r);
-    goff_k[u] = 8 * c < a.Dv ? (uint32_t)(r * a.kst * 2 + c * 16) : kNoRec;
-    goff_v[u] = 8 * c < a.Dv ? (uint32_t)(r * a.vst * 2 + c * 16) : kNoRec;
+    goff_k[u] = 8 * c < Dv ? (uint32_t)(r * a.kst * 2 + c * 16) : kNoRec;
+    goff_v[u] = 8 * c < Dv ? (uint32_t)(r * a.vst * 2 + c * 16) : kNoRec;
   }
   auto tile_rs = [&](const T* base, int64_t st, int t) __attribute__((always_inline)) {
     const int rows = min(Tk - t * BN, BN);
-    const uint32_t nrec = rows > 0 ? (uint32_t)((int64_t)(rows - 1) * st * 2 + 2 * a.Dv) : 0u;
+    const uint32_t nrec = rows > 0 ? (uint32_t)((int64_t)(rows - 1) * st * 2 + 2 * Dv) : 0u;
     return __builtin_amdgcn_make_buffer_rsrc((void*)(base + (rows > 0 ? (int64_t)t * BN * st : 0)), (short)0,
                                              (int)nrec, 0x00020000);
   };
@@ -974,29 +985,29 @@ __global__ __launch_bounds__(256, 1) void dq_wide_kernel(const BwdArgs a) {
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
     const int idx = lane + u * 64, r = idx / CH, c = idx % CH;
-    if (q0w + r < Tq && 8 * c < a.Dv) gstore16(dqp + (int64_t)(q0w + r) * a.dqst + c * 8, ov[u]);
+    if (q0w + r < Tq && 8 * c < Dv) gstore16(dqp + (int64_t)(q0w + r) * a.dqst + c * 8, ov[u]);
   }
 }
 
-template <typename T, bool CAUSAL>
+template <typename T, bool CAUSAL, bool FULL>
 hipError_t launch_dq_w(const BwdArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)(a.B * a.Hq * a.nqt)), block(256);
   const bool m = a.mask != nullptr, sc = a.score != nullptr;
-  if (m && sc) hipLaunchKernelGGL((dq_wide_kernel<T, CAUSAL, true, true>), grid, block, 0, s, a);
-  else if (m) hipLaunchKernelGGL((dq_wide_kernel<T, CAUSAL, true, false>), grid, block, 0, s, a);
-  else if (sc) hipLaunchKernelGGL((dq_wide_kernel<T, CAUSAL, false, true>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((dq_wide_kernel<T, CAUSAL, false, false>), grid, block, 0, s, a);
+  if (m && sc) hipLaunchKernelGGL((dq_wide_kernel<T, CAUSAL, true, true, FULL>), grid, block, 0, s, a);
+  else if (m) hipLaunchKernelGGL((dq_wide_kernel<T, CAUSAL, true, false, FULL>), grid, block, 0, s, a);
+  else if (sc) hipLaunchKernelGGL((dq_wide_kernel<T, CAUSAL, false, true, FULL>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((dq_wide_kernel<T, CAUSAL, false, false, FULL>), grid, block, 0, s, a);
   return hipGetLastError();
 }
 
-template <typename T, bool CAUSAL>
+template <typename T, bool CAUSAL, bool FULL>
 hipError_t launch_fwd_w(const FwdArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)(a.B * a.Hq * a.nqt)), block(256);
   const bool m = a.mask != nullptr, sc = a.score != nullptr;
-  if (m && sc) hipLaunchKernelGGL((fwd_wide_kernel<T, CAUSAL, true, true>), grid, block, 0, s, a);
-  else if (m) hipLaunchKernelGGL((fwd_wide_kernel<T, CAUSAL, true, false>), grid, block, 0, s, a);
-  else if (sc) hipLaunchKernelGGL((fwd_wide_kernel<T, CAUSAL, false, true>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((fwd_wide_kernel<T, CAUSAL, false, false>), grid, block, 0, s, a);
+  if (m && sc) hipLaunchKernelGGL((fwd_wide_kernel<T, CAUSAL, true, true, FULL>), grid, block, 0, s, a);
+  else if (m) hipLaunchKernelGGL((fwd_wide_kernel<T, CAUSAL, true, false, FULL>), grid, block, 0, s, a);
+  else if (sc) hipLaunchKernelGGL((fwd_wide_kernel<T, CAUSAL, false, true, FULL>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((fwd_wide_kernel<T, CAUSAL, false, false, FULL>), grid, block, 0, s, a);
   return hipGetLastError();
 }
 
@@ -1018,6 +1029,18 @@ hipError_t launch_kv_both(const BwdArgs& a, hipStream_t s) {
 }
 
 template <typename T>
+hipError_t launch_fwd_c(const FwdArgs& a, bool causal, hipStream_t s) {
+  if (a.Dv == kWD) return causal ? launch_fwd_w<T, true, true>(a, s) : launch_fwd_w<T, false, true>(a, s);
+  return causal ? launch_fwd_w<T, true, false>(a, s) : launch_fwd_w<T, false, false>(a, s);
+}
+
+template <typename T>
+hipError_t launch_dq_c(const BwdArgs& a, bool causal, hipStream_t s) {
+  if (a.Dv == kWD) return causal ? launch_dq_w<T, true, true>(a, s) : launch_dq_w<T, false, true>(a, s);
+  return causal ? launch_dq_w<T, true, false>(a, s) : launch_dq_w<T, false, false>(a, s);
+}
+
+template <typename T>
 hipError_t launch_kv_c(const BwdArgs& a, bool causal, hipStream_t s) {
   if (a.Dv == kWD) return causal ? launch_kv_both<T, true, true>(a, s) : launch_kv_both<T, false, true>(a, s);
   return causal ? launch_kv_both<T, true, false>(a, s) : launch_kv_both<T, false, false>(a, s);
@@ -1029,14 +1052,12 @@ int fwd_wide_block_rows() { return kWRows; }
 int dq_wide_block_rows() { return kWDqRows; }
 
 hipError_t launch_bwd_dq_wide(const BwdArgs& a, int dtype, bool causal, hipStream_t s) {
-  if (dtype == 0) return causal ? launch_dq_w<bf16, true>(a, s) : launch_dq_w<bf16, false>(a, s);
-  return causal ? launch_dq_w<f16, true>(a, s) : launch_dq_w<f16, false>(a, s);
+  return dtype == 0 ? launch_dq_c<bf16>(a, causal, s) : launch_dq_c<f16>(a, causal, s);
 }
 int kv_wide_block_keys() { return kWKvKeys; }
 
 hipError_t launch_fwd_wide(const FwdArgs& a, int dtype, bool causal, hipStream_t s) {
-  if (dtype == 0) return causal ? launch_fwd_w<bf16, true>(a, s) : launch_fwd_w<bf16, false>(a, s);
-  return causal ? launch_fwd_w<f16, true>(a, s) : launch_fwd_w<f16, false>(a, s);
+  return dtype == 0 ? launch_fwd_c<bf16>(a, causal, s) : launch_fwd_c<f16>(a, causal, s);
 }
 
 hipError_t launch_bwd_kv_wide(const BwdArgs& a, int dtype, bool causal, hipStream_t s) {
