@@ -186,6 +186,7 @@ __global__ __launch_bounds__(kRWaves * 64, D == 256 ? 1 : 2) void fwd_rows_kerne
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb) oacc[nb] = f32x16{};
   float m_run = kNegInf, l_run = 0.f;
+  float m_lift = kNegInf;   // what a tile's maximum has to exceed to move m_run (with a score)
   const int tr_row = 4 * hf + ((lane >> 2) & 3);
   const int tr_col = ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
   char* vt = smem + wave * VT;
@@ -254,18 +255,18 @@ __global__ __launch_bounds__(kRWaves * 64, D == 256 ? 1 : 2) void fwd_rows_kerne
       for (int j = 1; j < 16; ++j) mx = fmaxf(mx, s[j]);
       mx = half_max(mx);
       const float mc = mx * c2;
-      if (wave_any(mc > m_run)) {
+      float mneg = m_run == kNegInf ? 0.f : -m_run;
+      if (wave_any(mc > (SCORE ? m_lift : m_run))) {   // (-inf for rows of far_max(): with every tile)
         const float m_new = m_run == kNegInf ? mc : raise_max(m_run, mc);
         const float alpha = m_run == kNegInf ? 0.f : exp2_fast(m_run - m_new);
         l_run *= alpha;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) oacc[nb] *= alpha;
         m_run = m_new;
-      }
-      float mneg = m_run == kNegInf ? 0.f : -m_run;
-      if constexpr (SCORE) {
-        const bool far = far_max(m_run) && mx > kNegInf;
-        if (wave_any(far)) {
+        mneg = m_run == kNegInf ? 0.f : -m_run;
+        if constexpr (SCORE) {
+          m_lift = far_max(m_run) ? kNegInf : m_run;
+          const bool far = far_max(m_run) && mx > kNegInf;
           const float sub = far ? mx : 0.f;
 #pragma unroll
           for (int j = 0; j < 16; ++j) s[j] -= sub;

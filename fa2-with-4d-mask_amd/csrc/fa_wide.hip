@@ -213,6 +213,7 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdArgs a) {
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb) oacc[nb] = f32x16{};
   float m_run = kNegInf, l_run = 0.f;
+  float m_lift = kNegInf;   // what a tile's maximum has to exceed to move m_run (with a score)
   // transpose-read lane pattern: rows 4 hf + (lane / 4) % 4 (+8), columns
   // 16 ((lane / 16) % 2) + 4 (lane % 4) of each 32-column block
   const int tr_row = 4 * hf + ((lane >> 2) & 3);
@@ -313,18 +314,19 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdArgs a) {
     // rescale (O in AGPRs, read, scaled and written back) is rare.
     mx = half_max(mx);
     const float mt = mx * c2;   // the row's largest logit of tile j (scaled)
-    if (wave_any(mt > m_run + kWLift)) {
+    // (Rows of far_max() come here with every tile: their m_lift is -inf.)
+    float mneg = m_run == kNegInf ? 0.f : -m_run;
+    if (wave_any(mt > (SCORE ? m_lift : m_run + kWLift))) {
       const float m_new = fmaxf(m_run, mt);
       const float alpha = m_run == kNegInf ? 0.f : exp2_fast(m_run - m_new);
       l_run *= alpha;
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) oacc[nb] *= alpha;
       m_run = m_new;
-    }
-    float mneg = m_run == kNegInf ? 0.f : -m_run;
-    if constexpr (SCORE) {
-      const bool far = far_max(m_run) && mx > kNegInf;
-      if (wave_any(far)) {
+      mneg = m_run == kNegInf ? 0.f : -m_run;
+      if constexpr (SCORE) {
+        m_lift = far_max(m_run) ? kNegInf : m_run + kWLift;
+        const bool far = far_max(m_run) && mx > kNegInf;
         const float sub = far ? mx : 0.f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) s_cur[i] -= sub;
