@@ -355,15 +355,21 @@ int choose_split(const FaBwdParams* p) {
 // a split adds 6 plus the fp32 partials' way to memory and back.  Tq 512, Tk
 // 8192, Hq 32, D 128: 169 us in one range, 82 in four (102 in two, 101 in six);
 // Tq 1024, Tk 1024, Hq 16: 30 in one, 35-47 in two to eight.
-int fwd_key_split(int64_t base, int64_t nt, int64_t rows, int D, bool prec) {
-  if (base >= kCus) return 1;
+//
+// `shared`: the causal head-dim-64 blocks of 128 rows, three per CU, which overlap
+// little: a block alone takes 0.76 a tile, a CU's blocks together 0.63 a tile, and a
+// head's blocks walk half of nt tiles on average.  Measured / estimated, in one, two,
+// three, four ranges: T 4096, Hq 8 58 45 43 45 / 57 45 44 47; T 2048, Hq 16 32 34 33
+// 34 / 32 33 34 37; T 1000, Hq 32 19 26 28 31 / 20 26 29 32.
+int fwd_key_split(int64_t base, int64_t nt, int64_t rows, int D, bool prec, bool shared) {
+  if (base >= (shared ? 3 : 1) * kCus) return 1;
   const double tile = D == 64 ? (prec ? 1.9 : 1.1) : (prec ? 2.7 : 1.7);
   int best = 1;
   double best_us = 0;
   for (int ns = 1; ns <= 16 && ns <= nt; ++ns) {
-    const int64_t wgs = base * ns, rounds = (wgs + kCus - 1) / kCus;
+    const int64_t wgs = base * ns, rounds = (wgs + kCus - 1) / kCus, nt_r = (nt + ns - 1) / ns;
     const double clk = 0.75 + 0.25 * std::min(1.0, (double)wgs / kCus);
-    double us = rounds * (8 + clk * tile * ((nt + ns - 1) / ns));
+    double us = shared ? 8 + std::max(0.76 * nt_r, 0.63 * base * nt / 2 / kCus) : rounds * (8 + clk * tile * nt_r);
     if (ns > 1) us += 6 + 1.5e-6 * rows * ns * D;
     if (ns == 1 || us < best_us) {
       best = ns;
@@ -401,7 +407,7 @@ FwdPlan fwd_plan(const FaFwdParams* p) {
     const int brows = fa::fwd_block_rows(p->head_dim, p->is_causal != 0, p->mask != nullptr, p->score != nullptr);
     const int64_t base = (int64_t)p->batch * p->heads_q * ((p->seqlen_q + brows - 1) / brows);
     const int64_t nt = (keys + fa::kFwdKeys - 1) / fa::kFwdKeys;
-    f.split = fwd_key_split(base, nt, rows, p->head_dim, p->mask || p->score);
+    f.split = fwd_key_split(base, nt, rows, p->head_dim, p->mask || p->score, brows < fa::kFwdRows);
   }
   if (f.split > 1) f.bytes = rows * f.split * (p->head_dim + 2) * (int64_t)sizeof(float);
   return f;

@@ -536,3 +536,14 @@ def test_forward_plan(lib):
     assert plan(batch=64, seqlen_q=1, seqlen_k=4096) == (0, 1)
     # causal rows see no key past the last row
     assert plan(seqlen_q=4, seqlen_k=16384, is_causal=1) == (0, 1)
+
+
+def test_forward_plan_shared_cus(lib):
+    """Causal head-dim-64 blocks share a CU: split only where the longest block alone
+    takes longer than a CU's share of all."""
+    ext = _ext()
+    for heads, T, want in ((8, 4096, 3), (16, 2048, 1), (32, 1000, 1), (32, 4096, 1), (8, 512, 1)):
+        f = ext.FaFwdPlan()
+        p = fwd_params(head_dim=64, heads_q=heads, heads_k=8, seqlen_q=T, seqlen_k=T, is_causal=1)
+        assert lib.fa_fwd_plan(ctypes.byref(p), ctypes.byref(f)) == 0
+        assert (f.needs_mask_ws, f.key_split) == (1, want), (heads, T)
