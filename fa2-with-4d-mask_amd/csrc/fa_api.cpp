@@ -381,12 +381,29 @@ int fwd_key_split(int64_t base, int64_t nt, int64_t rows, int D, bool prec, bool
 // ---- how the forward runs ----------------------------------------------------
 // Few query rows: the rows of a kv-head's group packed into blocks of 32
 // (fa_rows.hip), which read the mask bytes themselves.  Its work grows with the
-// rows, that of a 256-row block does not, which meets at 64 rows, or 128 where
-// the prepared mask (16 us) is saved too.  Measured at Tk 16384, Hq 32, Hk 8, D
-// 128, in us, this kernel / the 256-row blocks with the key axis split: Tq 32
-// 33 / 63, Tq 64 50 / 65, Tq 128 84 / 68; with a mask Tq 64 61 / 110, Tq 128 104 /
-// 117, Tq 256 186 / 132.
-bool few_rows(const FaFwdParams* p) { return p->seqlen_q <= (p->mask ? 128 : 64); }
+// rows, that of a 256-row block (128 at head dim 256) does not.  Measured against
+// those blocks with the key axis split where it helps, bf16, this kernel / the
+// blocks, in us (`prepared`: the caller has the prepared mask, as a training step
+// does; otherwise the blocks need its launches first, 16 us and more):
+//   head dim 128, Hq 32, Hk 8        B1 Tk16384  B16 Tk4096  B64 Tk512  B64 Tk64
+//     no mask, Tq 64                    51 /  68   167 / 224  104 / 147   48 /  58
+//     mask, Tq 64                       65 / 113   201 / 349  122 / 215   56 /  79
+//     mask, Tq 96                       86 / 113   277 / 360  168 / 219   78 /  82
+//     mask, Tq 128                     103 / 117   364 / 369  221 / 232  100 /  85
+//     mask prepared, Tq 64              65 /  94   201 / 341  117 / 217   53 /  73
+//     mask prepared, Tq 128            104 / 101   365 / 360  250 / 235   99 /  81
+// so up to 64 rows; with a mask not yet prepared 96, or 128 while the blocks all
+// run at once.  At head dim 256 one workgroup fits a CU, whose tiles then cost as
+// much as a 128-row block's: B16 Hq16 Hk4 Tk4096, blocks of 32 rows 64 55 / 164, 128
+// 67 / 164, 256 92 / 172, 320 165 / 165, 512 182 / 169 (Tk64 21 / 12); so while they all
+// run at once, and, without a mask to prepare, with a tile for every wave (T 16
+// causal 9.7 / 8.2).
+int64_t few_rows_slots(const FaFwdParams* p) { return (p->head_dim > 128 ? 1 : 2) * kCus; }
+bool few_rows(const FaFwdParams* p, int64_t blocks, int64_t tiles) {
+  const bool bytes = p->mask && !p->mask_ws, once = blocks <= few_rows_slots(p);
+  if (p->seqlen_q > (bytes ? (once ? 128 : 96) : 64)) return false;
+  return p->head_dim <= 128 || (once && (bytes || tiles >= 4));
+}
 constexpr int kMaxKeySplit = 64;   // fwd_combine_kernel: one range per lane
 struct FwdPlan {
   bool rows;       // few-rows kernel
@@ -397,12 +414,13 @@ FwdPlan fwd_plan(const FaFwdParams* p) {
   FwdPlan f{false, 1, 0};
   const int64_t G = p->heads_q / p->heads_k, R = G * p->seqlen_q, rows = (int64_t)p->batch * p->heads_q * p->seqlen_q;
   const int64_t keys = p->is_causal ? std::min(p->seqlen_q, p->seqlen_k) : p->seqlen_k;
-  if (few_rows(p)) {
+  // few query rows: the rows of a kv-head's group in blocks of 32
+  const int64_t base32 = (int64_t)p->batch * p->heads_k * ((R + 31) / 32);
+  const int64_t nt32 = (keys + fa::fwd_rows_keys() - 1) / fa::fwd_rows_keys();
+  if (few_rows(p, base32, nt32)) {
     f.rows = true;
-    // two workgroups per CU; a range holds at least one tile per wave
-    const int64_t base = (int64_t)p->batch * p->heads_k * ((R + 31) / 32);
-    const int64_t nt = (keys + fa::fwd_rows_keys() - 1) / fa::fwd_rows_keys();
-    f.split = (int)std::max<int64_t>(1, std::min<int64_t>({2 * kCus / base, nt / 4, kMaxKeySplit}));
+    // as many ranges as workgroups fit on the chip; at least one tile per wave
+    f.split = (int)std::max<int64_t>(1, std::min<int64_t>({few_rows_slots(p) / base32, nt32 / 4, kMaxKeySplit}));
   } else if (p->head_dim <= 128) {
     const int brows = fa::fwd_block_rows(p->head_dim, p->is_causal != 0, p->mask != nullptr, p->score != nullptr);
     const int64_t base = (int64_t)p->batch * p->heads_q * ((p->seqlen_q + brows - 1) / brows);

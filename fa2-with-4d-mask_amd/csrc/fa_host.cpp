@@ -134,7 +134,9 @@ bool forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& ma
     p.score_stride_b = side_stride(score, 0); p.score_stride_h = side_stride(score, 1); p.score_stride_q = side_stride(score, 2);
   }
   FaFwdPlan plan{};
+  if (residual) p.mask_ws = p.mask;   // (for the plan: it will be prepared, the backward reads it)
   if (g_api.fwd_plan(&p, &plan) != FA_OK) return false;
+  p.mask_ws = nullptr;
   RECORD_FUNCTION("tilelang_fa2_4d_mask::fwd", c10::ArrayRef<const c10::IValue>());   // (the custom op's name in a profile)
 
   const auto bytes = q.options().dtype(at::kByte);

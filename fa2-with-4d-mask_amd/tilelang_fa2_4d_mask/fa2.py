@@ -279,7 +279,9 @@ def _forward_impl(q, k, v, Mask, Score, scale: float, is_causal: bool, residual:
             p.stream = _stream(q.device)
             lib = _ext.load_library()
             plan = _ext.FaFwdPlan()
+            p.mask_ws = p.mask if residual else None   # for the plan: it will be prepared, the backward reads it
             _ext.check(lib.fa_fwd_plan(ctypes.byref(p), ctypes.byref(plan)), "fa_fwd_plan", lib)
+            p.mask_ws = None
             if plan.workspace_bytes:
                 ws = torch.empty((plan.workspace_bytes,), dtype=torch.uint8, device=q.device)
                 p.workspace, p.workspace_bytes = ws.data_ptr(), plan.workspace_bytes

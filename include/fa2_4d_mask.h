@@ -73,7 +73,9 @@ typedef struct FaFwdParams {
   int32_t dtype;                 /* enum FaDtype */
   void* stream;                  /* hipStream_t; NULL = default stream */
   const void* mask_ws;           /* prepared mask (fa_mask_prepare of this mask); required with a mask unless
-                                    fa_fwd_plan says that the launch reads the mask itself */
+                                    fa_fwd_plan says that the launch reads the mask itself.  fa_fwd_plan looks
+                                    only at whether it is NULL: give any other value there when the mask is
+                                    prepared in any case (a backward follows), and fa_fwd the workspace then */
   void* o_lo;                    /* optional [B, Tq, Hq, D] dtype output, written with a mask or a score only:
                                     O's rounding residual (O in fp32 minus O as stored, rounded to dtype),
                                     for fa_bwd_preprocess; NULL = not written */
@@ -204,7 +206,7 @@ int fa_mask_prepare(const FaMaskParams* p);
 int fa_fwd(const FaFwdParams* p);
 
 /* Fills *plan for the problem in *p (no launch, no GPU access): sizes, head dim,
- * dtype, causality, and whether mask / score are non-NULL. */
+ * dtype, causality, and whether mask / score / mask_ws are non-NULL. */
 int fa_fwd_plan(const FaFwdParams* p, FaFwdPlan* plan);
 
 /* Backward preprocess.  Replaces `bwd_preprocess` (python/fa2.py:142-179, launched at

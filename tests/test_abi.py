@@ -547,3 +547,30 @@ def test_forward_plan_shared_cus(lib):
         p = fwd_params(head_dim=64, heads_q=heads, heads_k=8, seqlen_q=T, seqlen_k=T, is_causal=1)
         assert lib.fa_fwd_plan(ctypes.byref(p), ctypes.byref(f)) == 0
         assert (f.needs_mask_ws, f.key_split) == (1, want), (heads, T)
+
+
+def test_forward_plan_routes(lib):
+    """The few-rows kernel only where it is the faster one: with a mask that is
+    prepared anyway up to 64 rows, at full grids up to 96, at head dim 256 only
+    while its workgroups (one per CU) all run at once and have a tile per wave."""
+    ext = _ext()
+
+    def plan(**kw):
+        f = ext.FaFwdPlan()
+        assert lib.fa_fwd_plan(ctypes.byref(fwd_params(**kw)), ctypes.byref(f)) == 0
+        return f.needs_mask_ws, f.key_split
+
+    few = lambda **kw: plan(**kw)[0] == 0
+    for Tq, prepared, batch, want in ((64, True, 1, True), (65, True, 1, False), (128, False, 1, True), (129, False, 1, False),
+                                      (64, True, 64, True), (96, False, 64, True), (97, False, 64, False),
+                                      (65, True, 64, False)):
+        kw = {"mask_ws": FAKE} if prepared else {}
+        assert few(batch=batch, seqlen_q=Tq, seqlen_k=4096, mask=FAKE, **kw) == want, (Tq, prepared, batch)
+    wide = dict(head_dim=256, heads_q=16, heads_k=4, seqlen_k=4096)
+    assert plan(batch=16, seqlen_q=16, **wide) == (0, 2)       # 128 workgroups of 32 rows: twice that fit
+    assert plan(batch=16, seqlen_q=32, **wide) == (0, 1)
+    assert not few(batch=16, seqlen_q=33, **wide) and not few(batch=16, seqlen_q=33, mask=FAKE, **wide)
+    assert few(seqlen_q=128, mask=FAKE, **wide)
+    wide["seqlen_k"] = 96
+    assert not few(seqlen_q=1, **wide) and few(seqlen_q=1, mask=FAKE, **wide)
+    assert not few(seqlen_q=1, mask=FAKE, mask_ws=FAKE, **wide)
