@@ -7,7 +7,8 @@ mask or a score the rounding of P before P V, which moves O by at most
 u sum(p |v|) / sum(p) <= u max|v|; with either P enters in two parts
 (u^2 max|v|); 2^-18 max|v| for fp32 sums, exp2 and the merges' factors.  In fp16
 the parts of a small p are subnormal (steps of 2^-24, so off by 2^-25 each, and
-sum(p) >= 1/2 as the running maximum exceeds no row's by more than one step):
+sum(p) >= 1/2 as the running maximum exceeds no row's by more than one step; for
+large negative scores see test_gpu_running_max.py):
 2^-24 sum|v| more.  LSE (base 2): fp32 dot products of D
 16-bit values, |dlogit| <= D 2^-24 sum|q k| scale log2e < 2e-4 here.
 """
@@ -64,6 +65,10 @@ def _check(seed, B, Hq, Hk, D, Tq, Tk, dtype, causal, mask, score, scale, residu
     with torch.no_grad():
         O, L, ws, lo = torch.ops.tilelang_fa2_4d_mask.fwd(*dv, scale, causal, False, residual)
     torch.cuda.synchronize()
+    _compare(O, L, lo if residual else None, q, k, v, m, s, scale, causal, dtype)
+
+
+def _compare(O, L, lo, q, k, v, m, s, scale, causal, dtype):
     bhsd = [x.transpose(1, 2).double() for x in (q, k, v)]
     ref = E.eager_ref(*bhsd, m, s, scale=scale, is_causal=causal, compute_dtype=torch.float64).transpose(1, 2)
     O = O.double().cpu()
@@ -75,7 +80,7 @@ def _check(seed, B, Hq, Hk, D, Tq, Tk, dtype, causal, mask, score, scale, residu
     sub = 2.0 ** -24 * (1 + v.float().abs().sum(1).max().item()) if dtype == torch.float16 else 0.0
     bound = u * ref.abs() + ((u * u if two else u) + 2.0 ** -18) * vmax + sub
     assert bool(((O - ref).abs()[fin] <= bound[fin]).all()), (O - ref).abs()[fin].max().item()
-    if residual and two:
+    if lo is not None and two:
         both = (O + lo.double().cpu() - ref).abs()
         # O + residual: the rounding of O itself drops out
         assert bool((both[fin] <= (u * u * ref.abs() + (u * u + 2.0 ** -18) * vmax + sub)[fin]).all())
@@ -95,7 +100,7 @@ ROWS = [
     (1, 6, 2, 64, 11, 33, torch.float16, True, None, None, 0.125),        # 33 packed rows, causal
     (2, 4, 2, 128, 64, 64, torch.bfloat16, True, "bernoulli", "normal", 0.09),
     (4, 8, 2, 128, 1, 3001, torch.bfloat16, False, "left", None, 0.09),
-    (2, 4, 2, 64, 3, 4133, torch.bfloat16, False, "bernoulli", None, 0.125),   # over 32 tiles per wave
+    (2, 4, 2, 64, 3, 4133, torch.bfloat16, False, "bernoulli", None, 0.125),   # byte loads
     (1, 4, 2, 128, 128, 1000, torch.float16, False, "chunk", None, 0.09),
     (2, 4, 4, 128, 1, 2048, torch.bfloat16, False, None, "padding", 0.09),
     (1, 4, 2, 128, 5, 700, torch.bfloat16, False, "bernoulli", "normal", 0.0),
@@ -113,6 +118,66 @@ def test_few_rows(cuda, case, residual):
     assert plan.needs_mask_ws == 0
     print("case", case, "ranges", plan.key_split, flush=True)
     _check(1, *case, residual=residual)
+
+
+# All keys in one range, as large batches run: no workspace, so no split.  Then a wave
+# has over 32 tiles, what it looks at together: dead ones between live ones, a window
+# wholly dead before one that is live, and the next tile's loads beside the last
+# tile's work throughout.
+ONE_RANGE = [
+    # D mask score
+    (128, None, None),
+    (64, "bernoulli", None),
+    (128, "late", None),
+    (64, "late", "normal"),
+    (128, "gaps", None),
+    (256, "gaps", "normal"),
+    (128, None, "padding"),
+    (256, None, None),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", ONE_RANGE, ids=lambda c: f"D{c[0]}{c[1] or ''}{c[2] or ''}")
+def test_many_tiles_per_wave(cuda, case, dtype):
+    from tilelang_fa2_4d_mask import _ext
+
+    D, mask, score = case
+    B, Hq, Hk, Tq, Tk, scale = 2, 4, 2, 3, 4300, 0.1
+    tiles = -(-Tk // 32)
+    assert tiles > 4 * 32            # four waves take every fourth tile each
+    print("case", case, dtype, flush=True)
+    q, k, v, m, s = _inputs(6, B, Hq, Hk, D, Tq, Tk, dtype, mask, score)
+    if mask == "late":               # all of each wave's first window dead, for one batch entry
+        m = torch.ones((B, 1, Tq, Tk), dtype=torch.bool)
+        m[0, ..., : 4 * 32 * 32] = False
+    elif mask == "gaps":             # two of three tiles dead, and a window with one live tile
+        t = torch.arange(Tk) // 32
+        m = ((t % 3 == 1) & ((t < 64) | (t >= 128) | (t == 100))).expand(B, 1, Tq, Tk).contiguous()
+    dv = [None if x is None else x.to(cuda) for x in (q, k, v, m, s)]
+    O = torch.full((B, Tq, Hq, D), float("nan"), dtype=dtype, device=cuda)
+    L = torch.empty((B, Hq, Tq), device=cuda)
+    p = _ext.FaFwdParams()
+    p.q, p.k, p.v, p.mask, p.score = (_ext.ptr(x) for x in dv)
+    p.o, p.lse = O.data_ptr(), L.data_ptr()
+    for n, x in (("q", dv[0]), ("k", dv[1]), ("v", dv[2]), ("o", O)):
+        for a, st in zip("bth", x.stride()):
+            setattr(p, f"{n}_stride_{a}", st)
+    for n, x in (("mask", dv[3]), ("score", dv[4])):
+        if x is not None:
+            st = [0 if x.shape[i] == 1 else x.stride(i) for i in range(3)]
+            for a, v_ in zip("bhq", st):
+                setattr(p, f"{n}_stride_{a}", v_)
+    p.batch, p.seqlen_q, p.seqlen_k, p.heads_q, p.heads_k, p.head_dim = B, Tq, Tk, Hq, Hk, D
+    p.scale, p.dtype = scale, _ext.dtype_code(dtype)
+    p.stream = torch.cuda.current_stream().cuda_stream
+    lib = _ext.load_library()
+    plan = _ext.FaFwdPlan()
+    _ext.check(lib.fa_fwd_plan(ctypes.byref(p), ctypes.byref(plan)), "fa_fwd_plan", lib)
+    assert plan.needs_mask_ws == 0 and plan.key_split > 1
+    _ext.check(lib.fa_fwd(ctypes.byref(p)), "fa_fwd", lib)
+    torch.cuda.synchronize()
+    _compare(O, L, None, q, k, v, m, s, scale, False, dtype)
 
 
 SPLIT = [
