@@ -818,7 +818,12 @@ __global__ __launch_bounds__(kKvWaves * 64, 1) __attribute__((amdgpu_waves_per_e
   mfma_acc_drain();   // before the epilogue reads the AGPR accumulators
 
   // ---- epilogue: dK, dV (dV of a kv-head with a dead row is NaN) ---------------------
-  const auto& e = args_again<BwdArgs>();
+  // (with a mask or a score the loop wants the scalar registers; without, the loop's
+  // schedule is 1 % better with the arguments held)
+  const auto& e = [&]() -> const auto& {
+    if constexpr (PREC) return args_again<BwdArgs>();
+    else return a;
+  }();
   const float scale = e.scale;
   const bool dead = e.dead[b * e.Hk + kvh] != 0;
   const float nanv = __builtin_nanf("");
