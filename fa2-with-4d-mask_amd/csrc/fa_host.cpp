@@ -12,8 +12,11 @@
 // attention() returns None, the node's backward calls `general_backward`.
 #include <torch/extension.h>
 
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/record_function.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 
 #include <algorithm>
@@ -28,8 +31,8 @@ namespace {
 using at::Tensor;
 
 // Entry points of libfa2_4d_mask.so as the Python loader resolved them, and
-// the Python side: general_backward(...), and whether a backward is a plain one
-// (nothing traces, transforms or intercepts it, and no setting sends it there).
+// the Python side: general_backward(...), and the module whose settings send a
+// backward there.
 struct Api {
   int (*fwd_plan)(const FaFwdParams*, FaFwdPlan*);
   int (*fwd)(const FaFwdParams*);
@@ -42,7 +45,7 @@ struct Api {
 };
 Api g_api{};
 PyObject* g_general_backward = nullptr;   // callable, held for good
-PyObject* g_plain_backward = nullptr;     // callable
+PyObject* g_settings = nullptr;           // module fa2: _event_log, DS_LIMIT_BYTES
 int64_t g_ds_limit = 0;                   // the default limit
 
 // A dense device tensor that is its own memory: no batched, wrapped, negated,
@@ -297,9 +300,21 @@ Gradients general_backward(const Tensor& dout, const Tensor& q, const Tensor& k,
   return {std::get<0>(r), std::get<1>(r), std::get<2>(r)};
 }
 
-bool plain_backward() {
+// A backward that nothing traces, transforms or intercepts, and no setting that only
+// the Python host path honours (fa2.py _plain_eager, without its Python calls: through
+// them a small step took 6 us longer).
+bool plain_backward(const Tensor& dout) {
+  using K = c10::DispatchKey;
+  const auto* meta = torch::autograd::impl::get_autograd_meta(dout);
+  if (!plain(dout) || (meta && meta->fw_grad_) || at::GradMode::is_enabled() ||
+      c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::PythonTorchFunctionTLS::stack_len() > 0 ||
+      c10::impl::tls_is_dispatch_key_included(K::FuncTorchDynamicLayerFrontMode) ||
+      c10::impl::tls_is_dispatch_key_included(K::Tracer) || c10::impl::tls_is_dispatch_key_included(K::PythonDispatcher))
+    return false;
   pybind11::gil_scoped_acquire gil;
-  return pybind11::handle(g_plain_backward)().cast<bool>();
+  const pybind11::handle m(g_settings);
+  const pybind11::object log = m.attr("_event_log"), limit = m.attr("DS_LIMIT_BYTES");
+  return log.is_none() && limit.equal(pybind11::int_(0));
 }
 
 struct Attention : torch::autograd::Function<Attention> {
@@ -324,7 +339,7 @@ struct Attention : torch::autograd::Function<Attention> {
     const bool causal = flags & 1, atomic = flags >> 1 & 1, bhsd = flags >> 2 & 1;
     Gradients g;
     bool done = false;
-    if (plain(grads[0]) && !at::GradMode::is_enabled() && plain_backward()) {
+    if (plain_backward(grads[0])) {
       at::AutoDispatchBelowADInplaceOrView below;
       done = ::backward(grads[0], s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7], s[8], scale, causal, atomic, bhsd, &g);
     }
@@ -361,13 +376,13 @@ std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& 
   return Attention::apply(q, k, v, f, scale, causal, atomic, bhsd);
 }
 
-void init(const std::vector<uintptr_t>& fn, pybind11::object general, pybind11::object plain, int64_t ds_limit) {
+void init(const std::vector<uintptr_t>& fn, pybind11::object general, pybind11::object settings, int64_t ds_limit) {
   TORCH_CHECK(fn.size() == 8, "eight entry points expected");
   g_api = Api{(decltype(Api::fwd_plan))fn[0],     (decltype(Api::fwd))fn[1],  (decltype(Api::mask_plan))fn[2],
               (decltype(Api::mask_prepare))fn[3], (decltype(Api::bwd_plan))fn[4], (decltype(Api::bwd_preprocess))fn[5],
               (decltype(Api::bwd))fn[6],          (decltype(Api::bwd_finalize))fn[7]};
   g_general_backward = general.release().ptr();
-  g_plain_backward = plain.release().ptr();
+  g_settings = settings.release().ptr();
   g_ds_limit = ds_limit;
 }
 

@@ -162,7 +162,7 @@ def load_library(path: os.PathLike | None = None) -> ctypes.CDLL:
 _host = None
 
 
-def load_host(general_backward, plain_backward, ds_limit: int):
+def load_host(general_backward, settings, ds_limit: int):
     """Loads (once) and returns the native eager host path (csrc/fa_host.cpp),
     bound to the loaded library; raises RuntimeError if it is absent."""
     global _host
@@ -181,7 +181,7 @@ def load_host(general_backward, plain_backward, ds_limit: int):
             raise RuntimeError(f"{HOST_PATH}: ABI version {mod.ABI_VERSION} != {ABI_VERSION}, rebuild it")
         fns = (lib.fa_fwd_plan, lib.fa_fwd, lib.fa_mask_plan, lib.fa_mask_prepare, lib.fa_bwd_plan,
                lib.fa_bwd_preprocess, lib.fa_bwd, lib.fa_bwd_finalize)
-        mod.init([ctypes.cast(f, ctypes.c_void_p).value for f in fns], general_backward, plain_backward, ds_limit)
+        mod.init([ctypes.cast(f, ctypes.c_void_p).value for f in fns], general_backward, settings, ds_limit)
         _host = mod
         return mod
 

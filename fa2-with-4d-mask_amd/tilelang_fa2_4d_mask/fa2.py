@@ -36,6 +36,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import sys
 from typing import Optional
 
 import torch
@@ -460,12 +461,6 @@ def _plain_eager(*tensors) -> bool:
     return all(x is None or type(x) is torch.Tensor or type(x) is torch.nn.Parameter for x in tensors)
 
 
-def _plain_backward() -> bool:
-    """The same for a backward of the native path (whose node also looks at its
-    tensors), and no setting that only the Python host path honours."""
-    return DS_LIMIT_BYTES == 0 and _plain_eager()
-
-
 def flash_attention_with_4d_mask(Q, K, V, Mask=None, Score=None, scale=None, is_causal=False,
                                  use_atomic_backward=True, bhsd_input=True):
     """``flash_attention_with_4d_mask(Q, K, V, Mask, Score, scale, is_causal,
@@ -478,7 +473,7 @@ def flash_attention_with_4d_mask(Q, K, V, Mask=None, Score=None, scale=None, is_
     from . import ops
 
     if _plain_eager(Q, K, V, Mask, Score) and Q.is_cuda and Q.dim() == 4:
-        host = _ext.load_host(_general_backward, _plain_backward, DS_LIMIT_DEFAULT)
+        host = _ext.load_host(_general_backward, sys.modules[__name__], DS_LIMIT_DEFAULT)
         O = host.attention(Q, K, V, Mask, Score, float(Q.shape[3] ** -0.5 if scale is None else scale),
                            bool(is_causal), bool(use_atomic_backward), bool(bhsd_input))
         if O is not None:
