@@ -402,6 +402,7 @@ int64_t few_rows_slots(const FaFwdParams* p) { return (p->head_dim > 128 ? 1 : 2
 bool few_rows(const FaFwdParams* p, int64_t blocks, int64_t tiles) {
   const bool bytes = p->mask && !p->mask_ws, once = blocks <= few_rows_slots(p);
   if (p->seqlen_q > (bytes ? (once ? 128 : 96) : 64)) return false;
+  if (blocks >= 1LL << 23) return false;   // (a grid of up to three times the blocks': below 2^32 threads)
   return p->head_dim <= 128 || (once && (bytes || tiles >= 4));
 }
 constexpr int kMaxKeySplit = 64;   // fwd_combine_kernel: one range per lane

@@ -262,8 +262,8 @@ bool backward(const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor
   Tensor dq_acc, dk_acc, dv_acc, ds;
   if (plan.needs_dq_accum) dq_acc = at::empty({plan.dq_accum_elems}, f32);
   if (plan.dkv_accum_elems > 0) {
-    dk_acc = plan.dkv_accum_zeroed ? at::zeros({plan.dkv_accum_elems}, f32) : at::empty({plan.dkv_accum_elems}, f32);
-    dv_acc = plan.dkv_accum_zeroed ? at::zeros({plan.dkv_accum_elems}, f32) : at::empty({plan.dkv_accum_elems}, f32);
+    dk_acc = at::empty({plan.dkv_accum_elems}, f32);
+    dv_acc = at::empty({plan.dkv_accum_elems}, f32);
     p.dk_accum = dk_acc.data_ptr<float>();
     p.dv_accum = dv_acc.data_ptr<float>();
   }
