@@ -58,8 +58,8 @@ namespace {
 // Waves per workgroup (32 query rows each).  Causal at head dim 64 without a
 // mask or score: 4, three workgroups per CU (168 registers, 48 KB of LDS), whose
 // lengths even out better over the CUs than those of one 256-row block per CU:
-// Hq 16, T 2048 39 -> 32 us, Hq 32 Hk 8 T 8192 310 -> 292, B1 T 256 10.2 -> 8.8 (B2
-// T 1000 Hq 32 23.7 -> 24.4).  Not causal, 8 share each tile among twice the rows:
+// Hq 16, T 2048 39 -> 32 us, Hq 32 Hk 8 T 8192 310 -> 292, B1 T 256 9.6 -> 7.9 (B2
+// T 1000 Hq 32 24.4 -> 24.7, B4 T 512 Hq 32 16.2 -> 16.8).  Not causal, 8 share each tile among twice the rows:
 // MQA Tq 2048, Tk 16384 292 us against 300 with 4, Tq 512, Tk 8192 in key ranges 54
 // against 65.  With a mask the prepared lists are for 256 rows; at head dim 128
 // the two groups of the 8 alternate by design.

@@ -15,7 +15,8 @@
 //
 // What bounds it: reading K and V once.  A wave holds one whole tile of K and
 // of V in flight (16 KB at head dim 128) while it works on the one before, two
-// workgroups per CU, so about 128 KB per CU are on the way at any time.  K rows
+// workgroups per CU (head dim 256: one), so about 128 KB per CU are on the way at any
+// time.  K rows
 // go straight from memory into MFMA operand registers (S^T = K Q^T reads a K
 // row per lane); only V takes the way through LDS, in a region of each wave's
 // own (no barrier in the loop), for the transpose reads of O^T += V^T P^T.
@@ -29,8 +30,8 @@
 //
 // Measured (bf16, Hq 32, Hk 8, D 128): one row against 16384 keys 15 us + 5 for
 // the combine (67 MB of K and V; 330 us in fwd_kernel, 32 workgroups); a batch of
-// 16, 3001 keys, left padding up to half: 34 + 4 us (253 + 16 for the prepared
-// mask before), the live 150-190 MB at 4.5-5 TB/s.
+// 16, 3001 keys, left padding up to half: 31 + 4 us (253 + 16 for the prepared
+// mask before), the live 155 MB at 5.0 TB/s.
 #include "fa_common.h"
 #include "fa_kernels.h"
 
