@@ -384,7 +384,8 @@ int fwd_key_split(int64_t base, int64_t nt, int64_t rows, int D, bool prec, bool
 // rows, that of a 256-row block (128 at head dim 256) does not.  Measured against
 // those blocks with the key axis split where it helps, bf16, this kernel / the
 // blocks, in us (`prepared`: the caller has the prepared mask, as a training step
-// does; otherwise the blocks need its launches first, 16 us and more):
+// does, and its launches, 12-16 us in both, are not counted; otherwise the blocks
+// need them first):
 //   head dim 128, Hq 32, Hk 8        B1 Tk16384  B16 Tk4096  B64 Tk512  B64 Tk64
 //     no mask, Tq 64                    51 /  68   167 / 224  104 / 147   48 /  58
 //     mask, Tq 64                       65 / 113   201 / 349  122 / 215   56 /  79
